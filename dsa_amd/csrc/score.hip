@@ -12,6 +12,8 @@
 #include "status.hpp"
 #include "waveops.hpp"
 
+#include <algorithm>
+
 namespace dsa {
 namespace {
 
@@ -284,18 +286,22 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 4 ? 2 : 1) void dense_scores
 // ---------------------------------------------------------------------------
 // Multi-query (prefill) scoring: many query blocks against one shared key set.
 // A workgroup owns kPrefillQueries consecutive queries of one key set, one
-// per wave, and streams the key units they see through LDS: each 64-key unit
-// is loaded from memory once and scored for all four queries, instead of
-// once per query.  Rows are padded to kPrefillRow bytes so the 16 rows a lane
-// group reads fall on different banks.  With a causal limit the heaviest
-// query blocks are dispatched first.  One query per wave needs about half the
-// registers of two; a workgroup holds one wave per SIMD and two or three
-// workgroups share a CU, so one workgroup's barrier waits and its top-k
-// epilogue run under another's MFMAs (eight queries per workgroup, one
-// workgroup per CU, measured 5 us slower per C4 layer; two, 60 us slower).
+// per wave, and one of `splits` equal runs of the key units they see, which
+// it streams through LDS: each 64-key unit is loaded from memory once and
+// scored for all four queries, instead of once per query.  Rows are padded to
+// kPrefillRow bytes so the 16 rows a lane group reads fall on different
+// banks.  fp8 rows are widened to bf16 (exact) on their way into LDS and read
+// in the decode kernel's k order, so a key scores the same on either path.
+// With a causal limit the heaviest query blocks are dispatched first.  One
+// query per wave needs about half the registers of two; a workgroup holds one
+// wave per SIMD and two or three workgroups share a CU, so one workgroup's
+// barrier waits and its top-k epilogue run under another's MFMAs (eight
+// queries per workgroup, one workgroup per CU, measured 5 us slower per
+// 4096 x 4096 causal layer; two, 60 us slower).
 // ---------------------------------------------------------------------------
 constexpr int kPrefillQueries = 4;
 constexpr int kPrefillRow = 272;
+constexpr uint32_t kDropOffset = 0x80000000u;  // past every score row: the store is dropped
 
 // ---------------------------------------------------------------------------
 // Exact top-k of one query's score row at the end of the prefill kernel, with
@@ -548,69 +554,90 @@ __device__ __forceinline__ void mfma_valu_interleave() {
   }
 }
 
-template <class Tag, bool kTopK>
+template <class Tag, class KF, bool kTopK>
 __global__ __launch_bounds__(64 * kPrefillQueries, 2) void prefill_scores_kernel(DenseArgs a, int32_t qblocks,
-                                                                            int32_t keysets) {
+                                                                            int32_t keysets, int32_t splits) {
   constexpr int kThreads = 64 * kPrefillQueries;
   constexpr int kRowSplit = kThreads / 64;
-  constexpr int kRowBytesPer = 256 / kRowSplit;
+  constexpr int kRowBytesPer = KF::kRowBytes / kRowSplit;
   constexpr int kVecs = kRowBytesPer / 16;
+  constexpr int kLdsBytesPer = 256 / kRowSplit;  // rows are bf16 / f16 in LDS
   __shared__ __align__(16) uint8_t lds[2][64 * kPrefillRow];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15;
   const int g = lane >> 4;
-  const int qb = qblocks - 1 - (int)(blockIdx.x / keysets);  // heaviest first
-  const int64_t keyset = blockIdx.x % keysets;
+  const uint32_t split = blockIdx.x % (uint32_t)splits;
+  const uint32_t block = blockIdx.x / (uint32_t)splits;
+  const int qb = qblocks - 1 - (int)(block / (uint32_t)keysets);  // heaviest first
+  const int64_t keyset = block % (uint32_t)keysets;
   const int L = a.length;
   const int qpk = a.queries_per_keyset;
   auto visible = [&](int t) { return a.causal_offset >= 0 ? min(L, t + a.causal_offset + 1) : L; };
   const int t_last = min(qpk - 1, qb * kPrefillQueries + kPrefillQueries - 1);
+  // This workgroup's units [u_begin, u_end) of the block's `units`.
   const int units = (visible(t_last) + 63) >> 6;
+  const int per_split = (units + splits - 1) / splits;
+  const int u_begin = min((int)split * per_split, units);
+  const int u_end = min(u_begin + per_split, units);
 
   uint4 qa[4][4];
   float wr[4][4];
   const int t = qb * kPrefillQueries + wave;
   const bool active = t < qpk;
   const int64_t seq = keyset * qpk + (active ? t : 0);
-  load_dense_head_tiles<4, KeysB16::kNaturalK>(a.q + seq * a.q_stride, a.w + seq * a.w_stride, r, g, qa, wr);
+  load_dense_head_tiles<4, KF::kNaturalK>(a.q + seq * a.q_stride, a.w + seq * a.w_stride, r, g, qa, wr);
   const int vis = active ? visible(t) : 0;
   float* orow = a.out + seq * a.out_stride;
   const BufferRsrc orsrc = make_buffer(orow, active ? (uint32_t)L * 4u : 0u);
 
-  const BufferRsrc kr = make_buffer(a.keys + keyset * a.key_stride * KeysB16::kRowBytes,
-                                    (uint32_t)L * KeysB16::kRowBytes);
+  const BufferRsrc kr = make_buffer(a.keys + keyset * a.key_stride * KF::kRowBytes, (uint32_t)L * KF::kRowBytes);
+  const float* scales = KF::kScaled ? a.scales + keyset * a.scale_stride : nullptr;
   const int lrow = threadIdx.x / kRowSplit;
   const int lpart = threadIdx.x % kRowSplit;
   uint4 stage[kVecs];  // the next unit, in flight while this one is scored
   auto fetch = [&](int u) {
-    const uint32_t off = (uint32_t)(u * 64 + lrow) * KeysB16::kRowBytes + lpart * kRowBytesPer;
+    const uint32_t off = (uint32_t)(u * 64 + lrow) * KF::kRowBytes + lpart * kRowBytesPer;
 #pragma unroll
     for (int k = 0; k < kVecs; ++k) stage[k] = buffer_load_16(kr, off + 16 * k);
   };
   auto put = [&](int buf) {
-    uint8_t* dst = lds[buf] + lrow * kPrefillRow + lpart * kRowBytesPer;
+    uint8_t* dst = lds[buf] + lrow * kPrefillRow + lpart * kLdsBytesPer;
 #pragma unroll
-    for (int k = 0; k < kVecs; ++k) *reinterpret_cast<uint4*>(dst + 16 * k) = stage[k];
+    for (int k = 0; k < kLdsBytesPer / 16; ++k) {
+      uint4 v;
+      if constexpr (KF::kRowBytes == KeysB16::kRowBytes)
+        v = stage[k];
+      else
+        v = fp8x8_to_bf16x8((k & 1) ? make_uint2(stage[k >> 1].z, stage[k >> 1].w)
+                                    : make_uint2(stage[k >> 1].x, stage[k >> 1].y));
+      *reinterpret_cast<uint4*>(dst + 16 * k) = v;
+    }
   };
   auto read_tile = [&](const uint8_t* base, int tile, uint4 (&raw)[KeysB16::kRaw]) {
-    const uint8_t* row = base + (16 * tile + r) * kPrefillRow + g * 16;
+    const uint8_t* row = base + (16 * tile + r) * kPrefillRow;
 #pragma unroll
-    for (int c = 0; c < KeysB16::kRaw; ++c) raw[c] = *reinterpret_cast<const uint4*>(row + 64 * c);
+    for (int c = 0; c < KeysB16::kRaw; ++c)
+      raw[c] = *reinterpret_cast<const uint4*>(row + 2 * kstep_dims<KF::kNaturalK>(g, c));
   };
   // Stores are unconditional: the buffer bounds drop keys past L, every key
   // of an inactive query and the "previous unit" of the first iteration.
+  // A 64-key unit lies in one scale block; the scale of the unit whose tile 3
+  // is pending is fetched an iteration ahead of its store.
+  auto unit_scale = [&](int u) { return KF::kScaled ? scales[min(max(u, 0) * 64, L - 1) >> 7] : 1.f; };
+  float scale = unit_scale(u_begin);
   auto store_unit = [&](const float (&sp)[4], int u) {
-    const float score = unit_reduce(sp, g);
+    float score = unit_reduce(sp, g);
+    if constexpr (KF::kScaled) score *= scale;
     const int key = u * 64 + lane;
-    buffer_store_f32(orsrc, (uint32_t)key * 4u, key < vis ? score : -__builtin_inff());
+    buffer_store_f32(orsrc, u < u_begin ? kDropOffset : (uint32_t)key * 4u, key < vis ? score : -__builtin_inff());
   };
 
   // Every load is unconditional (a fetch past the last unit re-reads it), so
   // that the compiler counts the memory operations in flight exactly.
-  const int last_unit = max(units - 1, 0);
-  fetch(0);
-  put(0);
+  const int last_unit = max(u_end - 1, 0);
+  fetch(min(u_begin, last_unit));
+  put(u_begin & 1);
   // The query tiles, weights and first unit have landed.  Without this wait
   // the compiler sees the query loads in flight at the loop head and places
   // their waits inside the loop, where they also wait for each iteration's
@@ -623,7 +650,7 @@ __global__ __launch_bounds__(64 * kPrefillQueries, 2) void prefill_scores_kernel
   for (int m = 0; m < 4; ++m) acc1[m] = floatx4{0.f, 0.f, 0.f, 0.f};
   float sp[4] = {0.f, 0.f, 0.f, 0.f};
   uint4 rawA[KeysB16::kRaw], rawB[KeysB16::kRaw];
-  for (int u = 0; u < units; ++u) {
+  for (int u = u_begin; u < u_end; ++u) {
     fetch(min(u + 1, last_unit));
     // Keep the loads ahead of the scoring: left to itself the scheduler
     // sinks them to the put at the end of the iteration.
@@ -636,6 +663,7 @@ __global__ __launch_bounds__(64 * kPrefillQueries, 2) void prefill_scores_kernel
     sp[3] = tile_reduce<4>(wr, acc1);
     mfma_valu_interleave();
     store_unit(sp, u - 1);
+    if constexpr (KF::kScaled) scale = unit_scale(u);
     read_tile(base, 2, rawA);
     tile_mfma<Tag, 4, KeysB16>(qa, rawB, acc1);
     sp[0] = tile_reduce<4>(wr, acc0);
@@ -654,13 +682,14 @@ __global__ __launch_bounds__(64 * kPrefillQueries, 2) void prefill_scores_kernel
     put((u + 1) & 1);
     __syncthreads();
   }
-  if (units > 0) {
+  if (u_end > u_begin) {
     sp[3] = tile_reduce<4>(wr, acc1);
-    store_unit(sp, units - 1);
+    store_unit(sp, u_end - 1);
   }
-  // Keys past this workgroup's units are invisible to all of its queries.
+  // Keys past the block's units are invisible to all of its queries; the
+  // splits fill them in turn.
   if (active)
-    for (int key = units * 64 + lane; key < L; key += 64) orow[key] = -__builtin_inff();
+    for (int key = (units + (int)split) * 64 + lane; key < L; key += 64 * splits) orow[key] = -__builtin_inff();
   if constexpr (kTopK) {
     __shared__ __align__(16) uint32_t topk_scratch[kPrefillQueries][kTopKScratch];
     if (active) {
@@ -917,17 +946,33 @@ int launch_dense_m(DenseArgs a, int64_t sequences, hipStream_t stream, hipEvent_
   return check_launch("dense_scores_kernel");
 }
 
+// Runs of key units per query block.  A chunk of a few hundred queries over a
+// long context has too few query blocks to fill the CUs (three workgroups are
+// resident on each), so its units are cut into as many runs as bring the grid
+// to kPrefillGrid workgroups (two rounds of the resident 768: their ends
+// average out, and 512 x 32768 causal took 212 us against 225 us at 768 and
+// 217 us at 2304).  A run keeps at least kPrefillMinUnits units: below, the
+// query tiles each run loads again cost as much as its scoring (16 units
+// leave 16 x 10916 at 21 us against 13 us; 4 gain nothing).  One run per block
+// took 489, 472 and 159 us at 512 x 32768, 64 x 32768 and 16 x 10916; the
+// runs take 212, 36 and 13 us.
+constexpr int64_t kPrefillGrid = 1536;
+constexpr int64_t kPrefillMinUnits = 8;
+int32_t prefill_splits(int64_t blocks, int64_t length) {
+  const int64_t units = (length + 63) / 64;
+  return (int32_t)std::max<int64_t>(1, std::min(kPrefillGrid / blocks, units / kPrefillMinUnits));
+}
+
 template <class Tag, class KF>
 int launch_dense(const DenseArgs& a, int64_t sequences, hipStream_t stream) {
-  if constexpr (KF::kRowBytes == KeysB16::kRowBytes) {
-    if (!a.head_ids && a.head_count == kHeads && a.queries_per_keyset >= kPrefillQueries) {
-      const int64_t keysets = sequences / a.queries_per_keyset;
-      const int64_t qblocks = (a.queries_per_keyset + kPrefillQueries - 1) / kPrefillQueries;
-      if (keysets * a.queries_per_keyset == sequences && qblocks * keysets <= 0x7fffffffLL) {
-        hipLaunchKernelGGL((prefill_scores_kernel<Tag, false>), dim3((unsigned)(qblocks * keysets)),
-                           dim3(64 * kPrefillQueries), 0, stream, a, (int32_t)qblocks, (int32_t)keysets);
-        return check_launch("prefill_scores_kernel");
-      }
+  if (!a.head_ids && a.head_count == kHeads && a.queries_per_keyset >= kPrefillQueries) {
+    const int64_t keysets = sequences / a.queries_per_keyset;
+    const int64_t qblocks = (a.queries_per_keyset + kPrefillQueries - 1) / kPrefillQueries;
+    if (keysets * a.queries_per_keyset == sequences && qblocks * keysets <= 0x7fffffffLL) {
+      const int32_t splits = prefill_splits(qblocks * keysets, a.length);
+      hipLaunchKernelGGL((prefill_scores_kernel<Tag, KF, false>), dim3((unsigned)(qblocks * keysets * splits)),
+                         dim3(64 * kPrefillQueries), 0, stream, a, (int32_t)qblocks, (int32_t)keysets, splits);
+      return check_launch("prefill_scores_kernel");
     }
   }
   if (!a.head_ids && a.head_count == kHeads) return launch_dense_m<Tag, KF, 4, false>(a, sequences, stream);
@@ -1076,11 +1121,11 @@ extern "C" int dsa_score_queries_topk(const void* queries, int64_t q_stride, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)(qblocks * keysets));
   if (key_dtype == kBF16)
-    hipLaunchKernelGGL((prefill_scores_kernel<Bf16Tag, true>), grid, dim3(64 * kPrefillQueries), 0, s, a,
-                       (int32_t)qblocks, (int32_t)keysets);
+    hipLaunchKernelGGL((prefill_scores_kernel<Bf16Tag, KeysB16, true>), grid, dim3(64 * kPrefillQueries), 0, s, a,
+                       (int32_t)qblocks, (int32_t)keysets, 1);
   else
-    hipLaunchKernelGGL((prefill_scores_kernel<F16Tag, true>), grid, dim3(64 * kPrefillQueries), 0, s, a,
-                       (int32_t)qblocks, (int32_t)keysets);
+    hipLaunchKernelGGL((prefill_scores_kernel<F16Tag, KeysB16, true>), grid, dim3(64 * kPrefillQueries), 0, s, a,
+                       (int32_t)qblocks, (int32_t)keysets, 1);
   return check_launch("prefill_scores_kernel");
 }
 
