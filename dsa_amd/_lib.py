@@ -110,6 +110,9 @@ _SIGNATURES: dict[str, list] = {
     ],
     "dsa_project_rows": [_p, _i64, _i64, _p, _i32, _i64, _i64, _p, _i64, _p],
     "dsa_project_rows_pair": [_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p],
+    "dsa_encode_keys_rows": [_p, _i64, _i64, _i64, _p, _i32, _p, _p, _p, _i32, ctypes.c_float, _p, _i32,
+                             ctypes.c_float, _p, _i32, _i64, _p, _i64, _p],
+    "dsa_encode_queries_rows": [_p, _i64, _i64, _i64, _p, _i32, _p, _p, ctypes.c_float, ctypes.c_float, _p, _p, _p],
     "dsa_dim_sketch": [_p, _i64, _i32, _i32, _p, _i32, _i32, _i32, ctypes.c_float, _p, _i32, _p],
     "dsa_abs_max": [_p, _i64, _i32, _p, _p],
     "dsa_fake_quantize": [_p, _i64, _i32, _i32, ctypes.c_float, _p, _p, _p],

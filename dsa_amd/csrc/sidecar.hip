@@ -3,8 +3,8 @@
 // encode_keys is k_norm(wk(hidden)) then the non-interleaved RoPE on the
 // first rope_dim dims; encode_queries is the RoPE on each head of
 // wq(hidden), plus weights_proj(hidden) * (heads * head_dim)^-0.5.  The
-// projections are plain GEMMs left to the platform BLAS; everything after
-// them runs here in one pass per row, reading the projection once and
+// projections run in project.hip and gemm.hip; everything after them that
+// they do not fuse runs here in one pass per row, reading the projection once and
 // writing the encoded row straight to its destination (for keys, a KV-cache
 // row given per token), where the reference chains a LayerNorm, slices,
 // six elementwise products/sums and a concatenation.
@@ -15,6 +15,7 @@
 // computes in fp32 (biased variance, eps inside the rsqrt) and rounds once
 // to the row dtype.
 #include "common.hpp"
+#include "dsa_amd.h"
 #include "status.hpp"
 
 namespace dsa {
@@ -50,8 +51,9 @@ struct EncodeArgs {
   const int64_t* out_rows; // nullable: output row of each token (cache append)
   int64_t out_row_limit;   // rows of the output; a token whose row is outside is not written
   const int64_t* positions;  // [tokens]
-  const float* ln_weight;  // nullable (no LayerNorm) else [dim]
-  const float* ln_bias;    // [dim]
+  const void* ln_weight;  // nullable (no LayerNorm) else [dim], fp32 or bf16 (ln_bf16)
+  const void* ln_bias;    // [dim]
+  int32_t ln_bf16;
   float ln_eps;
   const float* w_in;       // nullable: [tokens][heads] fp32 head weights
   float* w_out;            // [tokens][heads]
@@ -130,6 +132,15 @@ __global__ __launch_bounds__(256) void encode_rows_kernel(EncodeArgs a) {
     for (int e = 0; e < 4; ++e)
       if (dim_of(e) >= dim) x[j][e] = 0.f;
 
+  float ln_w[4] = {}, ln_b[4] = {};
+  if (a.ln_weight)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = min(dim_of(e), dim - 1);
+      ln_w[e] = load_elem(a.ln_weight, d, a.ln_bf16);
+      ln_b[e] = load_elem(a.ln_bias, d, a.ln_bf16);
+    }
+
   const float pos = (float)a.positions[token];
   for (int i = lane; i < half; i += kWave) {
     // inv_freq_i = theta ^ (-i / half), angle = position * inv_freq_i (fp32).
@@ -165,7 +176,7 @@ __global__ __launch_bounds__(256) void encode_rows_kernel(EncodeArgs a) {
       for (int e = 0; e < 4; ++e) {
         const int d = dim_of(e);
         if (d < dim) {
-          const float v = __fadd_rn(__fmul_rn(__fmul_rn(y[e] - mean, rstd), a.ln_weight[d]), a.ln_bias[d]);
+          const float v = __fadd_rn(__fmul_rn(__fmul_rn(y[e] - mean, rstd), ln_w[e]), ln_b[e]);
           y[e] = out_bf16 ? round_bf16(v) : v;
         }
       }
@@ -282,11 +293,11 @@ extern "C" int dsa_rope(const void* x, void* out, const int64_t* positions, int6
   return launch_encode(a, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int dsa_encode_keys_epilogue(const void* proj, int32_t proj_dtype, int64_t proj_row_stride,
-                                        const float* ln_weight, const float* ln_bias, float ln_eps,
-                                        const int64_t* positions, int32_t rope_dim, float theta, void* out,
-                                        int32_t out_dtype, int64_t out_row_stride, const int64_t* out_rows,
-                                        int64_t out_row_limit, int64_t tokens, int32_t dim, void* stream) {
+static int encode_keys_epilogue(const void* proj, int32_t proj_dtype, int64_t proj_row_stride, const void* ln_weight,
+                                const void* ln_bias, int32_t ln_dtype, float ln_eps, const int64_t* positions,
+                                int32_t rope_dim, float theta, void* out, int32_t out_dtype, int64_t out_row_stride,
+                                const int64_t* out_rows, int64_t out_row_limit, int64_t tokens, int32_t dim,
+                                void* stream) {
   DSA_REQUIRE(ln_weight && ln_bias, "null pointer argument");
   EncodeArgs a = {};
   a.in = proj;
@@ -298,6 +309,7 @@ extern "C" int dsa_encode_keys_epilogue(const void* proj, int32_t proj_dtype, in
   a.positions = positions;
   a.ln_weight = ln_weight;
   a.ln_bias = ln_bias;
+  a.ln_bf16 = ln_dtype == kBF16;
   a.ln_eps = ln_eps;
   a.tokens = tokens;
   a.heads = 1;
@@ -309,6 +321,33 @@ extern "C" int dsa_encode_keys_epilogue(const void* proj, int32_t proj_dtype, in
   if (int st = check_encode(a, proj_dtype, out_dtype)) return st;
   DSA_REQUIRE(proj_row_stride >= dim && out_row_stride >= dim, "row strides must cover dim");
   return launch_encode(a, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dsa_encode_keys_epilogue(const void* proj, int32_t proj_dtype, int64_t proj_row_stride,
+                                        const float* ln_weight, const float* ln_bias, float ln_eps,
+                                        const int64_t* positions, int32_t rope_dim, float theta, void* out,
+                                        int32_t out_dtype, int64_t out_row_stride, const int64_t* out_rows,
+                                        int64_t out_row_limit, int64_t tokens, int32_t dim, void* stream) {
+  return encode_keys_epilogue(proj, proj_dtype, proj_row_stride, ln_weight, ln_bias, kF32, ln_eps, positions, rope_dim,
+                              theta, out, out_dtype, out_row_stride, out_rows, out_row_limit, tokens, dim, stream);
+}
+
+extern "C" int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim,
+                                    const void* wk, int32_t dim, void* proj, const void* ln_weight,
+                                    const void* ln_bias, int32_t ln_dtype, float ln_eps, const int64_t* positions,
+                                    int32_t rope_dim, float theta, void* out, int32_t out_dtype,
+                                    int64_t out_row_stride, const int64_t* out_rows, int64_t out_row_limit,
+                                    void* stream) {
+  DSA_REQUIRE(proj && ln_weight && ln_bias && positions && out, "null pointer argument");
+  DSA_REQUIRE(ln_dtype == kF32 || ln_dtype == kBF16, "the LayerNorm's weight and bias must be fp32 or bf16 (got %d)",
+              ln_dtype);
+  int st = tokens <= 16 && kdim % 32 == 0 && dim % 16 == 0
+               ? dsa_project_rows(hidden, hidden_stride, tokens, wk, kBF16, dim, kdim, proj, dim, stream)
+               : dsa_project_gemm(hidden, kBF16, hidden_stride, tokens, kdim, wk, kBF16, dim, proj, dim, 1.f, nullptr,
+                                  0.f, nullptr, 0, stream);
+  if (st) return st;
+  return encode_keys_epilogue(proj, kBF16, dim, ln_weight, ln_bias, ln_dtype, ln_eps, positions, rope_dim, theta, out,
+                              out_dtype, out_row_stride, out_rows, out_row_limit, tokens, dim, stream);
 }
 
 extern "C" int dsa_encode_queries_epilogue(const void* proj, const float* proj_weights, const int64_t* positions,

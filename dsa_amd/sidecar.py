@@ -174,6 +174,29 @@ def _token_positions(positions, shape, device) -> torch.Tensor:
     return pos.to(torch.int64).contiguous().reshape(-1)
 
 
+def _hidden_rows(hidden: torch.Tensor, tokens: int, kdim: int) -> torch.Tensor:
+    """hidden as ``[tokens, kdim]`` rows the projection kernels can read: unit
+    stride inside a row, rows 16-byte aligned."""
+
+    flat = hidden.reshape(tokens, kdim)
+    if flat.stride(-1) != 1 or (tokens > 1 and (flat.stride(0) % 8 or flat.stride(0) < kdim)) or flat.data_ptr() % 16:
+        flat = flat.contiguous()
+        if flat.data_ptr() % 16:
+            flat = flat.clone()
+    return flat
+
+
+def _cache_rows(out, out_rows, tokens: int, dim: int, device) -> torch.Tensor:
+    """The checked cache row of every token of ``encode_keys(out=...)``."""
+
+    if out.ndim != 2 or out.shape[1] != dim or not out.is_contiguous():
+        raise ValueError("out must be a contiguous [rows, head_dim] key cache")
+    if out_rows is None or out_rows.numel() != tokens:
+        raise ValueError("out_rows must give one cache row per token")
+    # (rows outside the cache are skipped by the kernel: no host sync here)
+    return out_rows.to(device=device, dtype=torch.int64).contiguous()
+
+
 def apply_noninterleaved_rope(x: torch.Tensor, positions: torch.Tensor, *, theta: float = 10_000.0) -> torch.Tensor:
     """Non-interleaved RoPE (reference sidecar.py:10-28) of x ``[..., d]``;
     positions has shape ``x.shape[:-1]`` or ``x.shape[:-2]`` (one position
@@ -336,6 +359,9 @@ class LightningIndexerSidecar(nn.Module):
 
         if not hidden.is_cuda:
             raise ValueError("HIP kernels require GPU tensors")
+        fused = self._encode_keys_rows(hidden, positions, out, out_rows)
+        if fused is not None:
+            return fused
         proj = self._project(hidden, self.wk.weight)
         tokens_shape = proj.shape[:-1]
         tokens = math.prod(tokens_shape)
@@ -348,12 +374,7 @@ class LightningIndexerSidecar(nn.Module):
             rows = None
             target = result
         else:
-            if out.ndim != 2 or out.shape[1] != self.head_dim or not out.is_contiguous():
-                raise ValueError("out must be a contiguous [rows, head_dim] key cache")
-            if out_rows is None or out_rows.numel() != tokens:
-                raise ValueError("out_rows must give one cache row per token")
-            # (rows outside the cache are skipped by the kernel: no host sync here)
-            rows = out_rows.to(device=hidden.device, dtype=torch.int64).contiguous()
+            rows = _cache_rows(out, out_rows, tokens, self.head_dim, hidden.device)
             target = out
         _lib.call(
             "dsa_encode_keys_epilogue", _lib.ptr(flat), _row_dtype(flat), self.head_dim, _lib.ptr(ln_w),
@@ -364,6 +385,60 @@ class LightningIndexerSidecar(nn.Module):
         if out is not None:
             return out
         return result.reshape(*tokens_shape, self.head_dim)
+
+    def _encode_keys_rows(self, hidden, positions, out, out_rows) -> torch.Tensor | None:
+        """:meth:`encode_keys` of bf16 hidden states with a bf16 wk in one
+        library call, which takes the LayerNorm's parameters as they are
+        stored; ``None`` where the separate calls are needed."""
+
+        weight, ln_w, ln_b = self.wk.weight, self.k_norm.weight, self.k_norm.bias
+        kdim, dim = hidden.shape[-1], self.head_dim
+        tokens = hidden.numel() // kdim if kdim else 0
+        if (tokens == 0 or hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
+                or weight.shape != (dim, kdim) or kdim % 8 or dim % 4 or ln_w.dtype != ln_b.dtype
+                or ln_w.dtype not in _ROW_DTYPES
+                or not (weight.is_cuda and weight.is_contiguous() and ln_w.is_contiguous() and ln_b.is_contiguous())):
+            return None
+        lead = hidden.shape[:-1]
+        pos = _token_positions(positions, lead, hidden.device)
+        if out is None:
+            target, rows = torch.empty((*lead, dim), device=hidden.device, dtype=torch.bfloat16), None
+            limit = tokens
+        else:
+            target, rows = out, _cache_rows(out, out_rows, tokens, dim, hidden.device)
+            limit = out.shape[0]
+        flat = _hidden_rows(hidden, tokens, kdim)
+        proj = torch.empty((tokens, dim), device=hidden.device, dtype=torch.bfloat16)
+        stride = flat.stride(0) if tokens > 1 else kdim
+        _lib.call("dsa_encode_keys_rows", flat.data_ptr(), stride, tokens, kdim, weight.data_ptr(), dim,
+                  proj.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), _ROW_DTYPES[ln_w.dtype], self.k_norm.eps,
+                  pos.data_ptr(), self.rope_dim, self.rope_theta, target.data_ptr(), _row_dtype(target), dim,
+                  _lib.ptr(rows), limit, _lib.stream_of(flat))
+        return target
+
+    def _encode_queries_rows(self, hidden, positions, scale) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """:meth:`encode_queries` of a decode step in one launch
+        (``dsa_encode_queries_rows``), identical to the separate calls;
+        ``None`` where those are needed."""
+
+        wq, wp = self.wq.weight, self.weights_proj.weight
+        kdim = hidden.shape[-1]
+        tokens = hidden.numel() // kdim if kdim else 0
+        if (not 0 < tokens <= 16 or kdim % 32 or hidden.dtype != torch.bfloat16 or wq.dtype != torch.bfloat16
+                or wp.dtype != torch.float32 or self.head_dim != HEAD_DIM or self.rope_dim != 64
+                or wq.shape != (self.heads * HEAD_DIM, kdim) or wp.shape != (self.heads, kdim)
+                or not (wq.is_cuda and wp.is_cuda and wq.is_contiguous() and wp.is_contiguous())):
+            return None
+        lead = hidden.shape[:-1]
+        pos = _token_positions(positions, lead, hidden.device)
+        flat = _hidden_rows(hidden, tokens, kdim)
+        queries = torch.empty((*lead, self.heads, HEAD_DIM), device=hidden.device, dtype=torch.bfloat16)
+        weights = torch.empty((*lead, self.heads), device=hidden.device, dtype=torch.float32)
+        stride = flat.stride(0) if tokens > 1 else kdim
+        _lib.call("dsa_encode_queries_rows", flat.data_ptr(), stride, tokens, kdim, wq.data_ptr(), self.heads,
+                  wp.data_ptr(), pos.data_ptr(), self.rope_theta, scale, queries.data_ptr(), weights.data_ptr(),
+                  _lib.stream_of(flat))
+        return queries, weights
 
     def encode_queries(self, hidden: torch.Tensor, positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """(queries ``[..., heads, head_dim]``, weights ``[..., heads]`` fp32)
@@ -382,6 +457,9 @@ class LightningIndexerSidecar(nn.Module):
             queries = self._project(hidden, self.wq.weight, positions=positions)
             weights = self._project(hidden, self.weights_proj.weight, fp32=True, scale=scale)
             return queries.reshape(*lead, self.heads, self.head_dim), weights.reshape(*lead, self.heads)
+        fused = self._encode_queries_rows(hidden, positions, scale)
+        if fused is not None:
+            return fused
         pair = self._project_pair(hidden, self.wq.weight, self.weights_proj.weight)
         if pair is None:
             proj = self._project(hidden, self.wq.weight)

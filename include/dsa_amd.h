@@ -781,6 +781,28 @@ int dsa_encode_queries_epilogue(const void* proj, const float* proj_weights, con
                                 float* out_weights, int64_t tokens, int32_t heads, int32_t dim,
                                 int32_t dtype, void* stream);
 
+/* encode_keys (sidecar.py:74-76) of bf16 hidden rows with a bf16 wk [dim][kdim]
+ * in one call: dsa_project_rows (at most 16 tokens, kdim a multiple of 32, dim
+ * of 16) or dsa_project_gemm into proj (bf16 [tokens][dim], scratch), then
+ * dsa_encode_keys_epilogue, with the LayerNorm's weight and bias in ln_dtype
+ * (DSA_DTYPE_F32 or DSA_DTYPE_BF16).  Results and limits are those calls'. */
+int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wk,
+                         int32_t dim, void* proj, const void* ln_weight, const void* ln_bias, int32_t ln_dtype,
+                         float ln_eps, const int64_t* positions, int32_t rope_dim, float theta, void* out,
+                         int32_t out_dtype, int64_t out_row_stride, const int64_t* out_rows, int64_t out_row_limit,
+                         void* stream);
+
+/* encode_queries (sidecar.py:78-88) of a decode step in one launch, for 1..16
+ * bf16 tokens, heads of 128 dims with the first 64 rotated: out_queries bf16
+ * [tokens][heads][128] = RoPE(hidden . wq^T), wq bf16 [heads * 128][kdim], and
+ * out_weights fp32 [tokens][heads] = (hidden . weights_proj^T) * weight_scale,
+ * weights_proj fp32 [heads][kdim].  Identical to dsa_project_rows_pair followed
+ * by dsa_encode_queries_epilogue; kdim a multiple of 32, hidden and wq 16-byte
+ * aligned. */
+int dsa_encode_queries_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wq,
+                            int32_t heads, const float* weights_proj, const int64_t* positions, float theta,
+                            float weight_scale, void* out_queries, float* out_weights, void* stream);
+
 /* ------------------------------------------------------------------------
  * Measurement utility (no counterpart in the reference; it serves the
  * roofline's measured peak): one launch that only reads `bytes` of device

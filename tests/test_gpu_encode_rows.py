@@ -1,0 +1,82 @@
+"""The encoders' single-call paths against the separate entry points they
+replace, bit for bit: dsa_encode_queries_rows (one launch for a decode step's
+wq with RoPE and weights_proj with its scale) against dsa_project_rows_pair
+and dsa_encode_queries_epilogue, and dsa_encode_keys_rows (LayerNorm
+parameters read as they are stored) against the projection and
+dsa_encode_keys_epilogue.  The separate entry points' parity with the oracle is
+test_gpu_sidecar.py's and test_gpu_sidecar_gemm.py's.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from dsa_amd import _lib, sidecar
+
+pytestmark = pytest.mark.gpu
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("tokens,kdim,heads,offset", [
+    (1, 32, 1, 0),      # one k-step: three quarters of k empty
+    (3, 96, 3, 0),      # an odd head count leaves half a weights_proj workgroup idle
+    (16, 2048, 64, 0),
+    (7, 2080, 64, 1),   # a second round of k, weights_proj 4-byte aligned only
+    (15, 4096, 5, 0),
+])
+def test_queries_equal_separate_calls(device, tokens, kdim, heads, offset) -> None:
+    print(f"encode queries rows tokens={tokens} kdim={kdim} heads={heads}", flush=True)
+    gen = torch.Generator().manual_seed(7 + kdim)
+    hidden = torch.randn(tokens, kdim + 8, generator=gen).to(device, torch.bfloat16)[:, :kdim]
+    wq = (torch.randn(heads * 128, kdim, generator=gen) * kdim**-0.5).to(device, torch.bfloat16)
+    wp = torch.randn(heads * kdim + offset, generator=gen).to(device)[offset:] * kdim**-0.5
+    if offset:
+        wp = torch.cat([torch.zeros(offset, device=device), wp])[offset:]
+        assert wp.data_ptr() % 16
+    positions = torch.randint(0, 40000, (tokens,), generator=gen).to(device)
+    scale = float((heads * 128) ** -0.5)
+    q = torch.empty(tokens, heads, 128, device=device, dtype=torch.bfloat16)
+    w = torch.empty(tokens, heads, device=device)
+    _lib.call("dsa_encode_queries_rows", hidden.data_ptr(), hidden.stride(0), tokens, kdim, wq.data_ptr(), heads,
+              wp.data_ptr(), positions.data_ptr(), 10000.0, scale, q.data_ptr(), w.data_ptr(), _stream())
+    pq, pw = torch.empty_like(q), torch.empty_like(w)
+    _lib.call("dsa_project_rows_pair", hidden.data_ptr(), hidden.stride(0), tokens, kdim, wq.data_ptr(), heads * 128,
+              pq.data_ptr(), heads * 128, wp.data_ptr(), heads, pw.data_ptr(), heads, _stream())
+    want_q, want_w = torch.empty_like(q), torch.empty_like(w)
+    _lib.call("dsa_encode_queries_epilogue", pq.data_ptr(), pw.data_ptr(), positions.data_ptr(), 64, 10000.0, scale,
+              want_q.data_ptr(), want_w.data_ptr(), tokens, heads, 128, _lib.DTYPE_BF16, _stream())
+    assert torch.equal(q.view(torch.int16), want_q.view(torch.int16))
+    assert torch.equal(w, want_w)
+
+
+@pytest.mark.parametrize("tokens,hidden_size,norm_dtype,cached", [
+    (1, 256, torch.bfloat16, True),
+    (16, 2048, torch.float32, False),
+    (13, 2048, torch.bfloat16, True),
+    (40, 264, torch.bfloat16, True),  # the GEMM path
+])
+def test_keys_equal_separate_calls(device, tokens, hidden_size, norm_dtype, cached) -> None:
+    print(f"encode keys rows tokens={tokens} hidden={hidden_size} norm={norm_dtype}", flush=True)
+    gen = torch.Generator().manual_seed(11 + tokens)
+    module = sidecar.LightningIndexerSidecar(hidden_size=hidden_size).to(device=device, dtype=torch.bfloat16).eval()
+    module.k_norm.to(norm_dtype)
+    with torch.no_grad():
+        module.k_norm.weight.copy_(1 + 0.1 * torch.randn(128, generator=gen))
+        module.k_norm.bias.copy_(0.1 * torch.randn(128, generator=gen))
+    hidden = torch.randn(tokens, hidden_size, generator=gen).to(device, torch.bfloat16)
+    positions = torch.randint(0, 40000, (tokens,), generator=gen).to(device)
+    rows = torch.randperm(64, generator=gen)[:tokens].to(device)
+    rows[-1] = 64  # outside the cache: not written
+    cache = torch.zeros(64, 128, device=device, dtype=torch.bfloat16)
+    got = module.encode_keys(hidden, positions, out=cache if cached else None, out_rows=rows if cached else None)
+    proj = module._project(hidden, module.wk.weight)
+    want = torch.zeros_like(cache) if cached else torch.empty(tokens, 128, device=device, dtype=torch.bfloat16)
+    ln_w, ln_b = module.k_norm.weight.detach().float(), module.k_norm.bias.detach().float()
+    _lib.call("dsa_encode_keys_epilogue", proj.data_ptr(), _lib.DTYPE_BF16, 128, ln_w.data_ptr(), ln_b.data_ptr(), 1e-6,
+              positions.data_ptr(), 64, 10000.0, want.data_ptr(), _lib.DTYPE_BF16, 128,
+              rows.data_ptr() if cached else None, want.shape[0], tokens, 128, _stream())
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
