@@ -110,9 +110,12 @@ _SIGNATURES: dict[str, list] = {
     ],
     "dsa_project_rows": [_p, _i64, _i64, _p, _i32, _i64, _i64, _p, _i64, _p],
     "dsa_project_rows_pair": [_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p],
-    "dsa_encode_keys_rows": [_p, _i64, _i64, _i64, _p, _i32, _p, _p, _p, _i32, ctypes.c_float, _p, _i32,
+    "dsa_encode_keys_rows": [_p, _i64, _i64, _i64, _p, _i32, _p, _i64, _p, _p, _i32, ctypes.c_float, _p, _i32,
                              ctypes.c_float, _p, _i32, _i64, _p, _i64, _p],
     "dsa_encode_queries_rows": [_p, _i64, _i64, _i64, _p, _i32, _p, _p, ctypes.c_float, ctypes.c_float, _p, _p, _p],
+    "dsa_project_weights": [_p, _i64, _i64, _i64, _p, _i64, ctypes.c_float, _p, _p, _i64, _p],
+    "dsa_encode_queries_gemm": [_p, _i64, _i64, _i64, _p, _i32, _p, _p, ctypes.c_float, ctypes.c_float, _p, _p, _p,
+                                _i64, _p],
     "dsa_dim_sketch": [_p, _i64, _i32, _i32, _p, _i32, _i32, _i32, ctypes.c_float, _p, _i32, _p],
     "dsa_abs_max": [_p, _i64, _i32, _p, _p],
     "dsa_fake_quantize": [_p, _i64, _i32, _i32, ctypes.c_float, _p, _p, _p],
@@ -124,6 +127,9 @@ _RESTYPES: dict[str, object] = {
     "dsa_temporal_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "dsa_topk_exact_workspace_bytes": (_i64, [_i64, _i64, _i32]),
     "dsa_project_gemm_workspace_bytes": (_i64, [_i64]),
+    "dsa_project_weights_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "dsa_encode_keys_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "dsa_encode_queries_workspace_bytes": (_i64, [_i64, _i64, _i64]),
 }
 
 

@@ -19,6 +19,13 @@
 #include "status.hpp"
 
 namespace dsa {
+
+// gemm.hip: the whole of encode_keys for batches of tokens.
+int launch_encode_keys_gemm(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wk,
+                            void* parts, const void* ln_weight, const void* ln_bias, bool ln_bf16, float ln_eps,
+                            const int64_t* positions, float theta, void* out, int64_t out_stride,
+                            const int64_t* out_rows, int64_t out_row_limit, hipStream_t stream);
+
 namespace {
 
 constexpr int kMaxRowDim = 256;  // dims per row a wave holds (4 per lane, in two adjacent pairs)
@@ -333,14 +340,28 @@ extern "C" int dsa_encode_keys_epilogue(const void* proj, int32_t proj_dtype, in
 }
 
 extern "C" int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim,
-                                    const void* wk, int32_t dim, void* proj, const void* ln_weight,
+                                    const void* wk, int32_t dim, void* workspace, int64_t workspace_bytes,
+                                    const void* ln_weight,
                                     const void* ln_bias, int32_t ln_dtype, float ln_eps, const int64_t* positions,
                                     int32_t rope_dim, float theta, void* out, int32_t out_dtype,
                                     int64_t out_row_stride, const int64_t* out_rows, int64_t out_row_limit,
                                     void* stream) {
-  DSA_REQUIRE(proj && ln_weight && ln_bias && positions && out, "null pointer argument");
+  DSA_REQUIRE(hidden && wk && ln_weight && ln_bias && positions && out, "null pointer argument");
   DSA_REQUIRE(ln_dtype == kF32 || ln_dtype == kBF16, "the LayerNorm's weight and bias must be fp32 or bf16 (got %d)",
               ln_dtype);
+  if (!workspace || workspace_bytes < dsa_encode_keys_workspace_bytes(tokens, kdim, dim) ||
+      reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+    return fail(DSA_STATUS_WORKSPACE_TOO_SMALL, "needs dsa_encode_keys_workspace_bytes(tokens, kdim, dim) bytes of "
+                                                "16-byte aligned workspace");
+  if (tokens > 16 && dim == kHeadDim && rope_dim == 64 && out_dtype == kBF16) {
+    DSA_REQUIRE(tokens <= 0x7fffffffLL && kdim > 0 && kdim % 8 == 0, "kdim %lld must be a positive multiple of 8",
+                (long long)kdim);
+    DSA_REQUIRE(out_row_stride >= dim, "row strides must cover dim");
+    return launch_encode_keys_gemm(hidden, hidden_stride, tokens, kdim, wk, workspace, ln_weight, ln_bias,
+                                   ln_dtype == kBF16, ln_eps, positions, theta, out, out_row_stride, out_rows,
+                                   out_rows ? out_row_limit : tokens, static_cast<hipStream_t>(stream));
+  }
+  void* proj = workspace;
   int st = tokens <= 16 && kdim % 32 == 0 && dim % 16 == 0
                ? dsa_project_rows(hidden, hidden_stride, tokens, wk, kBF16, dim, kdim, proj, dim, stream)
                : dsa_project_gemm(hidden, kBF16, hidden_stride, tokens, kdim, wk, kBF16, dim, proj, dim, 1.f, nullptr,

@@ -303,6 +303,12 @@ class LightningIndexerSidecar(nn.Module):
         if kdim % 8 or features % 4:
             raise ValueError("sidecar projections need a hidden width that is a multiple of 8 and a multiple of "
                              "4 output features")
+        if w.dtype == torch.float32 and hidden.dtype == torch.bfloat16 and positions is None:
+            need = int(_lib.query("dsa_project_weights_workspace_bytes", tokens, kdim, features))
+            ws = torch.empty(need, device=hidden.device, dtype=torch.uint8)
+            _lib.call("dsa_project_weights", _lib.ptr(flat), flat.stride(0), tokens, kdim, _lib.ptr(w), features,
+                      float(1.0 if scale is None else scale), _lib.ptr(out), _lib.ptr(ws), need, stream)
+            return out.reshape(*lead, features)
         pos = None
         ws = None
         need = 0
@@ -408,10 +414,11 @@ class LightningIndexerSidecar(nn.Module):
             target, rows = out, _cache_rows(out, out_rows, tokens, dim, hidden.device)
             limit = out.shape[0]
         flat = _hidden_rows(hidden, tokens, kdim)
-        proj = torch.empty((tokens, dim), device=hidden.device, dtype=torch.bfloat16)
+        need = int(_lib.query("dsa_encode_keys_workspace_bytes", tokens, kdim, dim))
+        ws = torch.empty(need, device=hidden.device, dtype=torch.uint8)
         stride = flat.stride(0) if tokens > 1 else kdim
         _lib.call("dsa_encode_keys_rows", flat.data_ptr(), stride, tokens, kdim, weight.data_ptr(), dim,
-                  proj.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), _ROW_DTYPES[ln_w.dtype], self.k_norm.eps,
+                  ws.data_ptr(), need, ln_w.data_ptr(), ln_b.data_ptr(), _ROW_DTYPES[ln_w.dtype], self.k_norm.eps,
                   pos.data_ptr(), self.rope_dim, self.rope_theta, target.data_ptr(), _row_dtype(target), dim,
                   _lib.ptr(rows), limit, _lib.stream_of(flat))
         return target
@@ -440,6 +447,29 @@ class LightningIndexerSidecar(nn.Module):
                   _lib.stream_of(flat))
         return queries, weights
 
+    def _encode_queries_gemm(self, hidden, positions, scale, tokens) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """:meth:`encode_queries` of a batch of bf16 tokens in one library
+        call (``dsa_encode_queries_gemm``); ``None`` where the separate calls
+        are needed."""
+
+        wq, wp = self.wq.weight, self.weights_proj.weight
+        kdim = hidden.shape[-1]
+        if (wp.dtype != torch.float32 or self.heads % 4 or wq.shape != (self.heads * HEAD_DIM, kdim)
+                or wp.shape != (self.heads, kdim)
+                or not (wq.is_cuda and wp.is_cuda and wq.is_contiguous() and wp.is_contiguous())):
+            return None
+        lead = hidden.shape[:-1]
+        pos = _token_positions(positions, lead, hidden.device)
+        flat = _hidden_rows(hidden, tokens, kdim)
+        queries = torch.empty((*lead, self.heads, HEAD_DIM), device=hidden.device, dtype=torch.bfloat16)
+        weights = torch.empty((*lead, self.heads), device=hidden.device, dtype=torch.float32)
+        need = int(_lib.query("dsa_encode_queries_workspace_bytes", tokens, kdim, self.heads))
+        ws = torch.empty(need, device=hidden.device, dtype=torch.uint8)
+        _lib.call("dsa_encode_queries_gemm", flat.data_ptr(), flat.stride(0), tokens, kdim, wq.data_ptr(), self.heads,
+                  wp.data_ptr(), pos.data_ptr(), self.rope_theta, scale, queries.data_ptr(), weights.data_ptr(),
+                  ws.data_ptr(), need, _lib.stream_of(flat))
+        return queries, weights
+
     def encode_queries(self, hidden: torch.Tensor, positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """(queries ``[..., heads, head_dim]``, weights ``[..., heads]`` fp32)
         (sidecar.py:78-88)."""
@@ -453,6 +483,9 @@ class LightningIndexerSidecar(nn.Module):
                 and hidden.shape[-1] % 8 == 0):
             # The RoPE of every head in the wq GEMM's output stage and the
             # head-weight scale in weights_proj's: no epilogue pass.
+            fused = self._encode_queries_gemm(hidden, positions, scale, tokens)
+            if fused is not None:
+                return fused
             lead = hidden.shape[:-1]
             queries = self._project(hidden, self.wq.weight, positions=positions)
             weights = self._project(hidden, self.weights_proj.weight, fp32=True, scale=scale)

@@ -782,15 +782,19 @@ int dsa_encode_queries_epilogue(const void* proj, const float* proj_weights, con
                                 int32_t dtype, void* stream);
 
 /* encode_keys (sidecar.py:74-76) of bf16 hidden rows with a bf16 wk [dim][kdim]
- * in one call: dsa_project_rows (at most 16 tokens, kdim a multiple of 32, dim
- * of 16) or dsa_project_gemm into proj (bf16 [tokens][dim], scratch), then
- * dsa_encode_keys_epilogue, with the LayerNorm's weight and bias in ln_dtype
- * (DSA_DTYPE_F32 or DSA_DTYPE_BF16).  Results and limits are those calls'. */
+ * in one call, with the LayerNorm's weight and bias in ln_dtype
+ * (DSA_DTYPE_F32 or DSA_DTYPE_BF16).  More than 16 tokens of 128 dims, 64 of
+ * them rotated, with a bf16 out: partial sums of wk over runs of k, then the
+ * rows from their sums.  Otherwise dsa_project_rows (at most 16 tokens, kdim a
+ * multiple of 32, dim of 16) or dsa_project_gemm, then
+ * dsa_encode_keys_epilogue.  Limits are those calls'; workspace (16-byte
+ * aligned) holds dsa_encode_keys_workspace_bytes(tokens, kdim, dim). */
+int64_t dsa_encode_keys_workspace_bytes(int64_t tokens, int64_t kdim, int64_t dim);
 int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wk,
-                         int32_t dim, void* proj, const void* ln_weight, const void* ln_bias, int32_t ln_dtype,
-                         float ln_eps, const int64_t* positions, int32_t rope_dim, float theta, void* out,
-                         int32_t out_dtype, int64_t out_row_stride, const int64_t* out_rows, int64_t out_row_limit,
-                         void* stream);
+                         int32_t dim, void* workspace, int64_t workspace_bytes, const void* ln_weight,
+                         const void* ln_bias, int32_t ln_dtype, float ln_eps, const int64_t* positions,
+                         int32_t rope_dim, float theta, void* out, int32_t out_dtype, int64_t out_row_stride,
+                         const int64_t* out_rows, int64_t out_row_limit, void* stream);
 
 /* encode_queries (sidecar.py:78-88) of a decode step in one launch, for 1..16
  * bf16 tokens, heads of 128 dims with the first 64 rotated: out_queries bf16
@@ -802,6 +806,28 @@ int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, int64_t toke
 int dsa_encode_queries_rows(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wq,
                             int32_t heads, const float* weights_proj, const int64_t* positions, float theta,
                             float weight_scale, void* out_queries, float* out_weights, void* stream);
+
+/* weights_proj (sidecar.py:55-58) of bf16 hidden rows for batches of tokens:
+ * out fp32 [tokens][features] = (hidden . weight) * scale, weight fp32
+ * [features][kdim], as partial sums over runs of k and their sums.  features a
+ * multiple of 4, kdim and hidden_stride of 8, pointers 16-byte aligned,
+ * dsa_project_weights_workspace_bytes of workspace. */
+int64_t dsa_project_weights_workspace_bytes(int64_t tokens, int64_t kdim, int64_t features);
+int dsa_project_weights(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const float* weight,
+                        int64_t features, float scale, float* out, void* workspace, int64_t workspace_bytes,
+                        void* stream);
+
+/* dsa_encode_queries_rows for any token count: weights_proj's partial sums over runs of k
+ * with the rotation table beside them, their sums, then dsa_project_gemm's
+ * rotated wq product.  Equal to dsa_project_gemm with positions and to
+ * dsa_project_weights; heads a multiple of 4,
+ * dsa_encode_queries_workspace_bytes(tokens, kdim, heads) of workspace, other
+ * limits dsa_project_gemm's, out_weights 16-byte aligned. */
+int64_t dsa_encode_queries_workspace_bytes(int64_t tokens, int64_t kdim, int64_t heads);
+int dsa_encode_queries_gemm(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim, const void* wq,
+                            int32_t heads, const float* weights_proj, const int64_t* positions, float theta,
+                            float weight_scale, void* out_queries, float* out_weights, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Measurement utility (no counterpart in the reference; it serves the
