@@ -1,8 +1,10 @@
 // Exact top-k with stable_topk semantics (reference metrics.py:9-22): the k
 // largest values, ties at the cut-off go to the lower index.
 //
-// One workgroup per (virtual) row: 1024 threads, or 256 when many short rows
-// (at most 4096 entries) make throughput matter more than latency.  Thread t owns the contiguous
+// One workgroup per (virtual) row.  topk_rows_kernel (1024 threads) takes plain
+// rows; topk_kernel takes many short rows (at most 4096 entries, 256 threads,
+// where throughput matters more than latency) and the merge of candidates
+// that carry their own indices (1024 threads).  In it, thread t owns the contiguous
 // slice [t * ept, t * ept + ept) of the row in registers (ept <= EPT, sized to
 // the row's length), so a single exclusive scan over threads enumerates
 // elements in index order.  The k-th
@@ -13,6 +15,7 @@
 #include "common.hpp"
 #include "select.hpp"
 #include "status.hpp"
+#include "waveops.hpp"
 
 namespace dsa {
 namespace {
@@ -424,6 +427,411 @@ __global__ __launch_bounds__(THREADS) void topk_kernel(TopkArgs a) {
   DSA_TRACE_MARK(g_trace_topk, blockIdx.x, 6);
 }
 
+// ---------------------------------------------------------------------------
+// The same selection, one 1024-thread workgroup per row, without per-element
+// scans: a bound on the cut, from a histogram of every element (of a quarter
+// of them on rows past 8192), leaves somewhat more than k candidates, which
+// are compacted in any order; the cut is resolved among them, and a bitmap of
+// the chosen positions brings the result into index order.
+//
+// topk_kernel passes over all of a row's elements five times (range, bins,
+// bin's members twice, slots), each thread owning a contiguous slice, so that
+// a load instruction of a wave touches 64 lines.  Here an element costs its
+// coalesced load, two range operations, one counter for every fourth one and
+// a compare with the bound; everything later is per candidate.
+//
+//  - Bins are linear in the order key between the row's least finite and its
+//    largest key: an eighth of an octave wide for scores around zero, finer
+//    for scores that share an offset, and monotone, so the bound (a bin's
+//    lower edge) never splits equal keys.
+//  - The sample's rank is k / 4 + 4 sqrt(k / 4) + 4, four and a half standard
+//    deviations above the quarter of the top k it holds on average: when it
+//    still leaves fewer than k candidates, or a crowded bin leaves more than
+//    fit, the row takes the radix select over all elements.
+//  - Up to 128 candidates are ranked against each other.  More are binned
+//    again, linearly in the key from the bound up, which leaves a few in a
+//    bin: in index order, the cut's bin is resolved by ranking its members; a
+//    sorted result is a counting sort by bin whose members order themselves.
+//    A bin of more than 64 leaves the row to the radix select.
+//
+// 512 rows of 32768, k = 2048, index order: 68 us -> 32.5 us (two rounds of
+// one workgroup per CU: 128 registers past 16384 elements); 100 rows of 16384:
+// 16.9 -> 11.0; one row of 32768, k = 2048, sorted: 42.5 -> 14.9 us, of 4096:
+// 26.5 -> 10.1 us (the bitonic sort took 66 barriers).
+// ---------------------------------------------------------------------------
+constexpr int kRowBins = 4096;
+constexpr int kRowPairs = 128;       // candidates ranked pairwise
+constexpr uint32_t kNegInfKey = 0x007fffffu;  // float_to_ordered(-inf)
+
+template <int CAP>
+struct RowShared {
+  uint64_t cand[CAP];
+  __align__(16) uint32_t bins[kRowBins];
+  uint32_t bits[kTopkThreads];   // chosen positions, 32 per word
+  uint32_t rank[kRowPairs];
+  uint64_t near[kWave];
+  __align__(16) uint32_t ws[2][kTopkThreads / kWave];
+  uint32_t wave_lo[kTopkThreads / kWave];
+  uint32_t wave_hi[kTopkThreads / kWave];
+  uint32_t digit, rem, count, near_n;
+  uint64_t cstar;
+};
+
+// Inclusive scans of 64 lanes by DPP for the minimum and maximum; the value
+// of the whole wave is read off the four row ends.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x111, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x112, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x114, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x118, 0xf, 0xf, false));
+  return min(min((uint32_t)__builtin_amdgcn_readlane(x, 15), (uint32_t)__builtin_amdgcn_readlane(x, 31)),
+             min((uint32_t)__builtin_amdgcn_readlane(x, 47), (uint32_t)__builtin_amdgcn_readlane(x, 63)));
+}
+
+// Shift that brings keys up to `span` above their origin into kRowBins bins.
+__device__ __forceinline__ int bin_shift(uint32_t span) { return max(0, 20 - (int)__clz((int)(span | 1u))); }
+
+template <int EPT, int CAP>
+__global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) void topk_rows_kernel(TopkArgs a) {
+  constexpr int kWaves = kTopkThreads / kWave;
+  constexpr int kStep = 4 * kTopkThreads;  // elements per load instruction of the workgroup
+  constexpr bool kSample = EPT > 8;
+  __shared__ RowShared<CAP> sh;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Last virtual rows first: under causal row lengths they are the longest.
+  const int64_t v = (int64_t)gridDim.x - 1 - blockIdx.x;
+  const int64_t row = v / a.chunks;
+  if (a.skip && a.skip[row]) return;
+  int row_len = a.length;
+  if (a.row_lengths) row_len = min(row_len, max(0, a.row_lengths[row]));
+  const int start = (int)(v % a.chunks) * a.chunk_len;
+  const int n = max(0, min(a.chunk_len, row_len - start));
+  const float* scores = a.scores + row * a.row_stride + start;
+  const int k = a.k;
+  const int64_t out_base = v * (int64_t)k;
+
+  // Element e of a thread is position kStep (e / 4) + 4 tid + e % 4; its order
+  // key, 0 past the row (the loads return 0 there).
+  uint32_t key[EPT];
+  auto pos_of = [&](int e) { return kStep * (e >> 2) + 4 * tid + (e & 3); };
+  {
+    const BufferRsrc rsrc = make_buffer(scores, (uint32_t)n * 4u);
+#pragma unroll
+    for (int c = 0; c < EPT / 4; ++c) {
+      uint4 raw = make_uint4(0u, 0u, 0u, 0u);
+      if (kStep * c < n) raw = buffer_load_16(rsrc, (uint32_t)(kStep * c + 4 * tid) * 4u);
+      key[4 * c + 0] = raw.x;
+      key[4 * c + 1] = raw.y;
+      key[4 * c + 2] = raw.z;
+      key[4 * c + 3] = raw.w;
+    }
+  }
+  reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+  sh.bits[tid] = 0;
+  if (tid < kRowPairs) sh.rank[tid] = 0;
+  if (tid == 0) sh.near_n = 0;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e)
+    key[e] = pos_of(e) < n ? float_to_ordered(__uint_as_float(key[e])) : 0u;
+
+  bool done = false;  // sorted output written
+  if (n <= k) {
+    // Every element is chosen.
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < EPT; e += 4)
+      if (pos_of(e) < n) {
+        const int left = min(4, n - pos_of(e));
+        atomicOr(&sh.bits[pos_of(e) >> 5], ((1u << left) - 1u) << (pos_of(e) & 31));
+      }
+  } else {
+    uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      lo = min(lo, key[e] > kNegInfKey ? key[e] : 0xffffffffu);
+      hi = max(hi, key[e]);
+    }
+    lo = wave_min_u32(lo);
+    hi = ~wave_min_u32(~hi);
+    if (lane == 0) {
+      sh.wave_lo[wave] = lo;
+      sh.wave_hi[wave] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      lo = min(lo, sh.wave_lo[i]);
+      hi = max(hi, sh.wave_hi[i]);
+    }
+    lo = min(lo, hi);
+    const int shift = bin_shift(hi - lo);
+#pragma unroll
+    for (int e = 0; e < EPT; e += kSample ? 4 : 1) {
+      if (kStep * (e >> 2) >= n) break;
+      if (pos_of(e) < n) lds_add(&sh.bins[key[e] <= lo ? 0u : (key[e] - lo) >> shift], 1u);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t want = (uint32_t)k;
+      if (kSample) {
+        const float quarter = 0.25f * (float)k;
+        want = min((uint32_t)(quarter + 4.f * sqrtf(quarter)) + 4u, (uint32_t)((n + 3) / 4));
+      }
+      const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, want, false);
+      if (lane == 0) sh.digit = loc.digit;
+    }
+    __syncthreads();
+    const uint32_t digit = sh.digit;
+    const uint32_t bound = digit == 0 ? 1u : lo + (digit << shift);
+    // Candidates: every key at or above the bound.
+    uint32_t mine = 0;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) mine += (uint32_t)__popcll(__ballot(key[e] >= bound));
+    if (lane == 0) sh.ws[0][wave] = mine;
+    reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    uint32_t at = 0, m = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      const uint32_t c = sh.ws[0][i];
+      at += i < wave ? c : 0u;
+      m += c;
+    }
+    at = __builtin_amdgcn_readfirstlane(at);
+    bool resolved = false;
+    if (m >= (uint32_t)k && m <= (uint32_t)CAP) {
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) {
+        const bool in = key[e] >= bound;
+        const uint64_t mask = __ballot(in);
+        if (in) sh.cand[at + lanes_below(mask)] = composite(key[e], pos_of(e));
+        at += (uint32_t)__popcll(mask);
+      }
+      __syncthreads();
+      if (m <= (uint32_t)kRowPairs) {
+        // Rank by pairwise comparison: `width` candidates, the threads past
+        // them each a further part of the comparisons.
+        int width = kWave;
+        while (width < (int)m) width <<= 1;
+        const int parts = kTopkThreads / width;
+        const int ci = tid & (width - 1);
+        const int per = ((int)m + parts - 1) / parts;
+        const int j0 = tid / width * per;
+        const int j1 = min((int)m, j0 + per);
+        const uint64_t c = sh.cand[min(ci, (int)m - 1)];
+        uint32_t larger = 0;
+#pragma unroll 8
+        for (int j = j0; j < j1; ++j) larger += sh.cand[j] > c ? 1u : 0u;
+        if (ci < (int)m) lds_add(&sh.rank[ci], larger);
+        __syncthreads();
+        if (tid < (int)m && sh.rank[tid] < (uint32_t)k) {
+          const uint64_t mine64 = sh.cand[tid];
+          const uint32_t p = ~(uint32_t)mine64;
+          if (a.sorted) {
+            const int64_t slot = out_base + sh.rank[tid];
+            if (a.out_idx) a.out_idx[slot] = start + (int64_t)p;
+            if (a.out_val) a.out_val[slot] = scores[p];
+          } else {
+            atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
+          }
+        }
+        done = a.sorted != 0;
+        resolved = true;
+      } else {
+        // Bins from the bound up, over the candidates alone.
+        const int shift2 = bin_shift(hi - bound);
+        uint64_t c[CAP / kTopkThreads];
+#pragma unroll
+        for (int i = 0; i < CAP / kTopkThreads; ++i) {
+          const int j = tid + kTopkThreads * i;
+          c[i] = j < (int)m ? sh.cand[j] : 0u;
+          if (c[i]) lds_add(&sh.bins[((uint32_t)(c[i] >> 32) - bound) >> shift2], 1u);
+        }
+        __syncthreads();
+        if (a.sorted) {
+          // Counting sort by bin, largest first; a bin's few members order
+          // themselves.  A crowded bin leaves the row to the radix select.
+          uint32_t b[4], sum = 0, most = 0;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            b[i] = sh.bins[kRowBins - 1 - 4 * tid - i];
+            sum += b[i];
+            most = max(most, b[i]);
+          }
+          if (most > (uint32_t)kWave) sh.near_n = 1;
+          uint32_t total;
+          uint32_t at2 = block_excl_scan<kWaves>(sum, sh.ws[1], total);
+          if (sh.near_n == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              sh.bins[kRowBins - 1 - 4 * tid - i] = at2;
+              at2 += b[i];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < CAP / kTopkThreads; ++i)
+              if (c[i]) sh.cand[atomicAdd(&sh.bins[((uint32_t)(c[i] >> 32) - bound) >> shift2], 1u)] = c[i];
+            __syncthreads();
+#pragma unroll 1
+            for (int j = tid; j < (int)m; j += kTopkThreads) {
+              const uint64_t x = sh.cand[j];
+              const uint32_t bin = ((uint32_t)(x >> 32) - bound) >> shift2;
+              int slot = j;
+              for (int q = j - 1; q >= 0; --q) {
+                const uint64_t y = sh.cand[q];
+                if (((uint32_t)(y >> 32) - bound) >> shift2 != bin) break;
+                slot -= y < x ? 1 : 0;
+              }
+              for (int q = j + 1; q < (int)m; ++q) {
+                const uint64_t y = sh.cand[q];
+                if (((uint32_t)(y >> 32) - bound) >> shift2 != bin) break;
+                slot += y > x ? 1 : 0;
+              }
+              if (slot < k) {
+                const uint32_t p = ~(uint32_t)x;
+                if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)p;
+                if (a.out_val) a.out_val[out_base + slot] = scores[p];
+              }
+            }
+            done = true;
+            resolved = true;
+          }
+        } else {
+          if (wave == 0) {
+            const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, (uint32_t)k, false);
+            if (lane == 0) {
+              sh.digit = loc.digit;
+              sh.rem = loc.rem;
+              sh.count = loc.count;
+            }
+          }
+          __syncthreads();
+        }
+        if (!a.sorted && sh.count <= (uint32_t)kWave) {
+          const uint32_t cut = sh.digit;
+#pragma unroll
+          for (int i = 0; i < CAP / kTopkThreads; ++i)
+            if (c[i] && ((uint32_t)(c[i] >> 32) - bound) >> shift2 == cut) sh.near[atomicAdd(&sh.near_n, 1u)] = c[i];
+          __syncthreads();
+          if (tid < (int)sh.count) {
+            const uint64_t x = sh.near[tid];
+            uint32_t larger = 0;
+            for (int j = 0; j < (int)sh.count; ++j) larger += sh.near[j] > x ? 1u : 0u;
+            if (larger + 1 == sh.rem) sh.cstar = x;
+          }
+          __syncthreads();
+          const uint64_t cstar = sh.cstar;
+#pragma unroll
+          for (int i = 0; i < CAP / kTopkThreads; ++i)
+            if (c[i] >= cstar && c[i]) {
+              const uint32_t p = ~(uint32_t)c[i];
+              atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
+            }
+          resolved = true;
+        }
+      }
+    }
+    if (!resolved) {
+      // Radix select of the k-th key over the whole row (12, 12 and 8 bits),
+      // then the ties at it in index order.
+      uint32_t prefix = 0, prefix_mask = 0, want = (uint32_t)k;
+#pragma unroll 1
+      for (int pass = 0; pass < 3; ++pass) {
+        const int sft = pass == 0 ? 20 : (pass == 1 ? 8 : 0);
+        const uint32_t dmask = pass == 2 ? 0xffu : 0xfffu;
+        __syncthreads();
+        reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < EPT; ++e)
+          if (key[e] != 0 && (key[e] & prefix_mask) == prefix) lds_add(&sh.bins[(key[e] >> sft) & dmask], 1u);
+        __syncthreads();
+        if (wave == 0) {
+          const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, want, false);
+          if (lane == 0) {
+            sh.digit = loc.digit;
+            sh.rem = loc.rem;
+          }
+        }
+        __syncthreads();
+        prefix |= sh.digit << sft;
+        prefix_mask |= dmask << sft;
+        want = sh.rem;
+      }
+      __syncthreads();
+      uint32_t* ties = sh.bins;  // one word per thread
+      ties[tid] = 0;
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) {
+        const int p = pos_of(e);
+        if (key[e] > prefix) atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
+        if (key[e] != 0 && key[e] == prefix) atomicOr(&ties[p >> 5], 1u << (p & 31));
+      }
+      __syncthreads();
+      uint32_t word = ties[tid];
+      uint32_t total;
+      const uint32_t before = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[0], total);
+      int take = (int)want - (int)before;  // this word's ties that are chosen, lowest first
+      uint32_t chosen = 0;
+      while (word && take > 0) {
+        chosen |= word & (0u - word);
+        word &= word - 1;
+        --take;
+      }
+      sh.bits[tid] |= chosen;
+    }
+  }
+  const int chosen_n = min(n, k);
+  if (!done) {
+    __syncthreads();
+    uint32_t word = sh.bits[tid];
+    uint32_t total;
+    uint32_t p = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[1], total);
+    // Exactly chosen_n bits are set; the bound only guards the buffers.
+    while (word) {
+      const uint32_t at = 32u * tid + (uint32_t)__builtin_ctz(word);
+      word &= word - 1;
+      if (p >= (uint32_t)chosen_n) break;
+      if (a.sorted) {
+        sh.cand[p] = composite(float_to_ordered(scores[at]), (int)at);
+      } else {
+        if (a.out_idx) a.out_idx[out_base + p] = start + (int64_t)at;
+        if (a.out_val) a.out_val[out_base + p] = scores[at];
+      }
+      ++p;
+    }
+    if (a.sorted) {
+      int width = 1;
+      while (width < chosen_n) width <<= 1;
+      for (int i = chosen_n + tid; i < width; i += kTopkThreads) sh.cand[i] = 0;
+      __syncthreads();
+      bitonic_sort_desc<kTopkThreads>(sh.cand, width);
+      for (int i = tid; i < chosen_n; i += kTopkThreads) {
+        const uint32_t at = ~(uint32_t)sh.cand[i];
+        if (a.out_idx) a.out_idx[out_base + i] = start + (int64_t)at;
+        if (a.out_val) a.out_val[out_base + i] = scores[at];
+      }
+    }
+  }
+  // Padding when the row has fewer than k elements.
+  for (int i = chosen_n + tid; i < k; i += kTopkThreads) {
+    if (a.out_idx) a.out_idx[out_base + i] = -1;
+    if (a.out_val) a.out_val[out_base + i] = -__builtin_inff();
+  }
+}
+
+template <int EPT>
+int launch_topk_rows_ept(const TopkArgs& a, dim3 grid, hipStream_t stream) {
+  if (a.k <= 2048)
+    hipLaunchKernelGGL((topk_rows_kernel<EPT, 4096>), grid, dim3(kTopkThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((topk_rows_kernel<EPT, 8192>), grid, dim3(kTopkThreads), 0, stream, a);
+  return check_launch("topk_rows_kernel");
+}
+
 int launch_topk(const TopkArgs& a, int64_t virtual_rows, hipStream_t stream) {
   const int n = a.chunk_len;
   const dim3 grid((unsigned)virtual_rows);
@@ -435,6 +843,12 @@ int launch_topk(const TopkArgs& a, int64_t virtual_rows, hipStream_t stream) {
     else if (n <= 256 * 8) hipLaunchKernelGGL((topk_kernel<256, 8, kSmallCap>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((topk_kernel<256, 16, kSmallCap>), grid, block, 0, stream, a);
     return check_launch("topk_kernel");
+  }
+  if (!a.in_idx) {
+    if (n <= kTopkThreads * 4) return launch_topk_rows_ept<4>(a, grid, stream);
+    if (n <= kTopkThreads * 8) return launch_topk_rows_ept<8>(a, grid, stream);
+    if (n <= kTopkThreads * 16) return launch_topk_rows_ept<16>(a, grid, stream);
+    return launch_topk_rows_ept<32>(a, grid, stream);
   }
   const dim3 block(kTopkThreads);
   if (n <= kTopkThreads * 4) hipLaunchKernelGGL((topk_kernel<kTopkThreads, 4, kMaxK>), grid, block, 0, stream, a);

@@ -1,0 +1,62 @@
+"""The one-workgroup row top-k (topk_rows_kernel through metrics.topk) against
+the oracle's stable_topk, bit for bit: the candidate bound from a full and from
+a sampled histogram, its pairwise, binned and radix resolutions, and the
+counting-sorted output, at the edges of the kernel's element counts and on rows
+whose scores share an offset, hold outliers, ties or -inf."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from dsa_amd import metrics
+from oracle import topk as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _row(kind: str, length: int, rng) -> np.ndarray:
+    x = rng.normal(size=length).astype(np.float32)
+    if kind == "offset":  # one binade: bins finer than the key's top bits
+        return (np.float32(100) + x * np.float32(0.01)).astype(np.float32)
+    if kind == "outlier":  # the range of two values hides the rest in a few bins
+        x[rng.integers(length)] = np.float32(1e30)
+        x[rng.integers(length)] = np.float32(-1e30)
+    elif kind == "tied":  # every cut crowded: the radix select and its ties
+        x = rng.integers(-2, 3, size=length).astype(np.float32)
+        x[x == 0] = rng.choice(np.array([0.0, -0.0], dtype=np.float32), size=int((x == 0).sum()))
+    elif kind == "equal":
+        x[:] = np.float32(-3.5)
+    elif kind == "sparse":  # fewer finite scores than k, and +inf
+        x[rng.random(length) < 0.97] = -np.inf
+        x[rng.integers(length)] = np.inf
+    elif kind == "periodic":  # the sampled quarter holds none of the top scores
+        x[np.arange(length) % 4 != 0] += np.float32(10)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "offset", "outlier", "tied", "equal", "sparse", "periodic"])
+@pytest.mark.parametrize("length,k", [(4095, 128), (4097, 130), (8192, 1), (8193, 2048), (16384, 2049), (16385, 100),
+                                      (30001, 4096), (32768, 600)])
+def test_rows_match_oracle(device, kind, length, k) -> None:
+    print(f"topk rows kind={kind} L={length} k={k}", flush=True)
+    rng = np.random.default_rng(length + k)
+    host = np.stack([_row(kind, length, rng) for _ in range(17)])  # 17 rows: past the distributed select
+    wide = torch.full((17, length + 3), float("inf"), device=device)
+    wide[:, :length] = torch.from_numpy(host)
+    x = wide[:, :length]
+    lengths = np.full(17, length, dtype=np.int32)
+    lengths[3], lengths[5], lengths[7], lengths[9] = 0, k, k + 1, length - 1
+    lens = torch.from_numpy(np.minimum(lengths, length)).to(device)
+    in_order, values = metrics.topk(x, k, sorted=False, row_lengths=lens, return_values=True)
+    ranked = metrics.topk(x, k, sorted=True, row_lengths=lens).cpu().numpy()
+    in_order, values = in_order.cpu().numpy(), values.cpu().numpy()
+    for r in (0, 3, 5, 7, 9, 16):
+        n = int(min(lengths[r], length))
+        assert ranked[r].tolist() == T.topk_sorted_padded(host[r], k, n).tolist(), r
+        want = T.topk_index_order(host[r], k, n)
+        assert in_order[r].tolist() == want.tolist(), r
+        chosen = want >= 0
+        np.testing.assert_array_equal(values[r][chosen].view(np.uint32), host[r][want[chosen]].view(np.uint32))
+        assert np.isneginf(values[r][~chosen]).all()
