@@ -21,10 +21,13 @@ from . import _lib
 
 MAX_K = 4096
 MAX_ROW = 32768
-# A few long rows in index order go through the distributed select (every CU
-# works on them) rather than one workgroup per row.
+# A few rows longer than one workgroup takes go, in index order, through the
+# distributed select (every CU works on them) rather than chunks and a merge.
+# Below, one workgroup per row is the faster: 1-16 rows of 16384, k 256 / 2048,
+# 9.8 / 11.0 us against 13.7 us, of 24001 12.6 / 13.8 against 13.9-14.9, of
+# 32768 13.5 / 14.9 against 13.6-15.3, and one launch against three.
 DISTRIBUTED_MAX_ROWS = 16
-DISTRIBUTED_MIN_LENGTH = 16384  # below, one workgroup per row is as fast (three launches cost more)
+DISTRIBUTED_MIN_LENGTH = MAX_ROW + 1
 DISTRIBUTED_MAX_LENGTH = 524288
 
 

@@ -152,6 +152,14 @@ def _weights_f32(weights: torch.Tensor) -> torch.Tensor:
     return weights.to(torch.float32).contiguous()
 
 
+def _threshold_on(device: torch.device, threshold: float | torch.Tensor) -> torch.Tensor:
+    """The promotion threshold as one fp32 value on the device."""
+
+    if isinstance(threshold, torch.Tensor) and threshold.dtype == torch.float32 and threshold.device == device:
+        return threshold.reshape(1)
+    return torch.as_tensor(threshold, device=device, dtype=torch.float32).reshape(1)
+
+
 def _head_ids_on(device: torch.device, ids: torch.Tensor) -> torch.Tensor:
     return ids.to(device=device, dtype=torch.int32).contiguous()
 
@@ -314,10 +322,11 @@ def progressive_scores_hip(
     keys = keys.contiguous()
     weights = _weights_f32(weights)
     direct = _mask_bytes(direct_full_blocks, keys.device)
-    threshold_tensor = torch.as_tensor(threshold, device=keys.device, dtype=torch.float32).reshape(1)
+    threshold_tensor = _threshold_on(keys.device, threshold)
     accepted = torch.empty(block_count, device=keys.device, dtype=torch.int8)
     block_max = torch.empty(block_count, device=keys.device, dtype=torch.float32)
-    counter = torch.zeros(1, device=keys.device, dtype=torch.int32)
+    # The candidate counter of compact output; the dense output needs none.
+    counter = torch.zeros(1, device=keys.device, dtype=torch.int32) if compact else None
     scores = torch.empty(length, device=keys.device, dtype=torch.float32)
     indices = torch.empty(length, device=keys.device, dtype=torch.int32) if compact else None
     _lib.call(
