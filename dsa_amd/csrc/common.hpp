@@ -109,6 +109,10 @@ __device__ __forceinline__ void buffer_store_16(BufferRsrc rsrc, uint32_t offset
   __builtin_amdgcn_raw_buffer_store_b128(parts, rsrc, (int)offset, 0, 0);
 }
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 buffer_load_8(BufferRsrc rsrc, uint32_t offset) {
+  const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)offset, 0, 0);
+  return make_uint2(v.x, v.y);
+}
 __device__ __forceinline__ void buffer_store_u64(BufferRsrc rsrc, uint32_t offset, uint64_t v) {
   const u32x2 parts = {(uint32_t)v, (uint32_t)(v >> 32)};
   __builtin_amdgcn_raw_buffer_store_b64(parts, rsrc, (int)offset, 0, 0);

@@ -59,7 +59,8 @@ struct DenseArgs {
   int32_t wgs_per_seq;
   int64_t total_wgs;  // the launch pads the grid to a multiple of kXcds
   uint32_t* hist;  // [sequences][kSelectBins] score histogram (kHist only)
-  // Candidate lists (kLists only): list (s, chunk) at lists[s * length + chunk * chunk_keys].
+  // Candidate lists (kLists only): list (s, chunk) at lists[s * length + chunk * chunk_keys],
+  // its scores, then its positions.
   uint64_t* lists;
   uint32_t* list_meta;  // [sequences][kMaxListChunks][2]: length, lowest bin listed
   int32_t list_quota;
@@ -260,8 +261,10 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 4 ? 2 : 1) void dense_scores
       __shared__ uint32_t s_list_bin;
       __shared__ __align__(16) uint32_t s_list_wsum[kWaves];
       write_chunk_list<kWaves>(hist, chunk_scores, chunk_keys, min(chunk_keys, valid - chunk_base), chunk_base,
-                               (uint32_t)a.list_quota, a.lists + seq * (int64_t)L + chunk_base,
-                               a.list_meta + 2 * (seq * kMaxListChunks + chunk), &s_list_bin, s_list_wsum);
+                               (uint32_t)a.list_quota,
+                               reinterpret_cast<uint32_t*>(a.lists + seq * (int64_t)L + chunk_base),
+                               min(chunk_keys, L - chunk_base), a.list_meta + 2 * (seq * kMaxListChunks + chunk), &s_list_bin,
+                               s_list_wsum);
       DSA_TRACE_MARK(g_trace_dense, blockIdx.x, 3);
       return;
     }

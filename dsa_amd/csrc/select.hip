@@ -435,20 +435,30 @@ __global__ __launch_bounds__(kSelThreads) void select_resolve_kernel(SelectArgs 
 // workgroup then writes its own list's chosen keys after the chosen keys of
 // the lists before it.
 //
-// Each list is read by threads_per_list consecutive threads (entry s by
-// thread s mod threads_per_list), whose first kListSpec entries are fetched
-// with the lists' lengths, in one round trip.
+// Each list is read by threads_per_list consecutive threads, four scores a
+// load (load q of thread r: entries 4 (r + threads_per_list q) on), the first
+// `loads` of them fetched with the lists' lengths, in one round trip.  That
+// covers twice the plan's quota: lists run past their quota by the rest of
+// its 12-bit bin, 1.2 to 1.9 times in all at 20,000 to 131,072 keys, and each
+// load more costs every workgroup 4 KB (32 single 8-byte entries a thread
+// took 0.7 us more than 24 at 20,011 keys).  Longer lists fetch the rest
+// once their lengths are there, up to kListVecs loads.
+//
+// Entries are compared as (score, place j * chunk_keys + s): the lists are in
+// index order, so places order as positions do, and only the workgroup's own
+// list's positions are read.
 // ---------------------------------------------------------------------------
-constexpr int kListSpec = 24;
+constexpr int kListVecs = 16;
 
 struct ListArgs {
   const float* scores;      // [rows, length]
-  const uint64_t* lists;    // [rows, length]: list j at j * chunk_keys
+  const uint64_t* lists;    // [rows, length]: list j at j * chunk_keys, scores then positions
   const uint32_t* meta;     // [rows][kMaxListChunks][2]: length, lowest bin listed
   int32_t length;
   int32_t chunks;           // lists per row
   int32_t chunk_keys;
   int32_t k;
+  int32_t loads;            // score loads per thread in the first round trip
   uint32_t total_wgs;       // rows * chunks (the grid is padded to a multiple of 8)
   int64_t* out_idx;         // [rows, k]
   float* out_val;           // [rows, k] or null
@@ -462,17 +472,205 @@ struct ListShared {
   uint64_t stage[kListStageCapacity];  // the row's entries, list j at base[j]
   uint64_t cands[kCandCapacity];       // the entries of the cut's bin
   RadixShared radix;
-  uint32_t hist[kSelectBins];  // bins of the entries; then the radix digit counters
+  alignas(16) uint32_t hist[kSelectBins];  // bins of the entries; then the radix digit counters
   uint32_t base[kMaxListChunks + 1];  // entry prefix over the row's sources
   uint32_t raw[kMaxListChunks];       // 1: the source is the chunk's raw scores
   uint32_t wsum[2][kSelWaves];
+  uint32_t wave_bin[kSelWaves], wave_len[kSelWaves];
   uint32_t bin, want, miss, crowd;
 };
 
+constexpr uint32_t kPastBuffer = 0xffffff00u;  // an offset past every buffer here: reads give 0
+
+// Four scores of a list from entry s on, or zeros without a fetch when s is
+// not below `limit` (a select, not a branch: loads under branches of their own
+// were waited for one by one); the buffer ends with the row's words, two per key, so a read
+// from an entry inside the list stays inside the row.
+__device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, uint32_t s, uint32_t limit) {
+  return buffer_load_16(words, s < limit ? (base + s) * 4u : kPastBuffer);
+}
+
+// ---------------------------------------------------------------------------
+// The usual case, with the entries in registers from the kernel's one round
+// trip of loads.  Every list holds all of its chunk's keys at or above
+// `origin`, the highest of the lists' lowest bins, so a k-th largest listed key
+// at or above it is the row's.  The entries are counted into bins of 2^11 keys
+// from there up, over an octave (above: the last bin): fine enough
+// that the cut's bin holds a few entries, so the entries of that bin, ranked
+// by every wave for itself, give the cut, where the 12-bit bins of the lists
+// leave 450 to 1,100 entries that took one or two more counting passes, and
+// whose counters serialised the first pass's atomics.  Five barriers in all.
+// Returns false, before anything is written, when a list is longer than the
+// registers hold, fewer than k keys lie at or above the origin (a list may
+// miss keys), or the cut lies past the octave or in a bin of more than 64
+// entries (ties).
+//
+// Bound by latency: the loads' round trip, five barriers and a few hundred
+// VALU instructions a wave, one wave per SIMD.  Counting the 12-bit bins and a
+// radix cut from 8-byte entries -> this, MI355X: 1 x 4096 k 256 6.6 -> 5.4 us;
+// 5 x 20011 k 2048 9.7 -> 7.3; 16 x 32768 k 2048 9.6 -> 7.0; 4 x 131072 k 2048
+// (fp8) 11.4 -> 7.5.  From 8-byte entries with these bins: 6.0, 6.8, 6.8, 8.8.
+// ---------------------------------------------------------------------------
+constexpr int kFineShift = 11;
+
+__device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared& sh, BufferRsrc words, uint32_t lbase,
+                                                  uint4 (&pre)[kListVecs], uint32_t list_len,
+                                                  uint32_t list_bin, uint32_t own_pos, uint32_t j, uint32_t r,
+                                                  uint32_t tpl, uint32_t row, uint32_t c) {
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = lane_id();
+  const uint32_t wave = tid / kWave;
+  const uint32_t kk = (uint32_t)a.k;
+  const uint32_t ck = (uint32_t)a.chunk_keys;
+#pragma unroll
+  for (int q = 0; q < kSelectBins / 4 / kSelThreads; ++q)
+    reinterpret_cast<uint4*>(sh.hist)[tid + kSelThreads * q] = make_uint4(0u, 0u, 0u, 0u);
+  if (tid == 0) sh.crowd = 0;
+  const uint32_t wbin = wave_max_u32(list_bin);  // (threads with no list read length and bin 0)
+  const uint32_t wlen = wave_max_u32(list_len);
+  if (lane == 0) {
+    sh.wave_bin[wave] = wbin;
+    sh.wave_len[wave] = wlen;
+  }
+  __syncthreads();
+  uint32_t top_bin = 0, longest = 0;
+#pragma unroll
+  for (int w = 0; w < kSelWaves; ++w) {
+    top_bin = max(top_bin, sh.wave_bin[w]);
+    longest = max(longest, sh.wave_len[w]);
+  }
+  if (longest > 4u * tpl * kListVecs) return false;
+  const int nq = __builtin_amdgcn_readfirstlane((int)((longest + 4u * tpl - 1u) / (4u * tpl)));
+  const uint32_t origin = top_bin << 20;
+  uint32_t* own_keys = reinterpret_cast<uint32_t*>(sh.stage);
+  // f(entry's place in its list, key) over this thread's loads; keys past the
+  // list's end read 0, which is below every key selected here.
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int q = 0; q < kListVecs; ++q) {
+      if (q < nq) {
+        const uint32_t s = 4u * (r + tpl * q);
+        f(s, pre[q].x);
+        f(s + 1u, pre[q].y);
+        f(s + 2u, pre[q].z);
+        f(s + 3u, pre[q].w);
+      }
+    }
+  };
+  if (nq > a.loads) {
+#pragma unroll
+    for (int q = 0; q < kListVecs; ++q)
+      if (q >= a.loads && q < nq) pre[q] = load_scores(words, lbase, 4u * (r + tpl * q), list_len);
+  }
+#pragma unroll
+  for (int q = 0; q < kListVecs; ++q) {
+    if (q < nq) {
+      const uint32_t s = 4u * (r + tpl * q);
+      const uint32_t left = list_len > s ? list_len - s : 0u;
+      pre[q].x = left > 0u ? pre[q].x : 0u;
+      pre[q].y = left > 1u ? pre[q].y : 0u;
+      pre[q].z = left > 2u ? pre[q].z : 0u;
+      pre[q].w = left > 3u ? pre[q].w : 0u;
+      if (j == c) *reinterpret_cast<uint4*>(own_keys + s) = pre[q];
+    }
+  }
+  if (j == c && r == 0) sh.base[0] = list_len;
+  each([&](uint32_t, uint32_t key) {
+    const uint32_t b = min((key - origin) >> kFineShift, (uint32_t)kSelectBins - 1u);
+    if (key >= max(origin, 1u))
+      __hip_atomic_fetch_add(&sh.hist[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  });
+  __syncthreads();
+  if (wave == 0) {
+    const Locate t = wave_locate<kSelectBins / kWave>(sh.hist, kk, false);
+    if (lane == 0) {
+      sh.bin = t.digit;
+      sh.want = t.rem;
+      sh.miss = t.count;
+    }
+  }
+  __syncthreads();
+  const uint32_t bin = sh.bin;
+  const uint32_t crowd = sh.miss;
+  if (bin >= (uint32_t)kSelectBins - 1u || crowd > (uint32_t)kWave) return false;  // (kNoBin is past every bin)
+  const uint32_t lowest = origin + (bin << kFineShift);
+  each([&](uint32_t s, uint32_t key) {
+    if (key - lowest < 1u << kFineShift && key != 0u)
+      sh.cands[__hip_atomic_fetch_add(&sh.crowd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)] =
+          select_composite(key, j * ck + s);
+  });
+  __syncthreads();
+  const uint64_t x = sh.cands[min(lane, crowd - 1u)];
+  uint32_t larger = 0;
+  for (uint32_t i = 0; i < crowd; ++i) larger += sh.cands[i] > x ? 1u : 0u;
+  const uint64_t hit = __ballot(lane < crowd && larger + 1u == sh.want);
+  const int owner = (int)__builtin_ctzll(hit);  // composites are distinct: one lane
+  const uint32_t cut = (uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), owner);
+  const uint32_t cut_place = ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, owner);
+  auto chosen = [&](uint32_t key, uint32_t place) { return key > cut || (key == cut && place <= cut_place); };
+  // Chosen entries of the lists before this one, and of this list in index
+  // order, a contiguous run per thread.
+  uint32_t before = 0;
+  if (j < c)
+    each([&](uint32_t s, uint32_t key) { before += chosen(key, j * ck + s) ? 1u : 0u; });
+  const uint32_t own_n = sh.base[0];
+  const uint32_t per = (own_n + kSelThreads - 1) / kSelThreads;
+  const uint32_t first = min(own_n, tid * per);
+  const uint32_t last = min(own_n, first + per);
+  uint32_t mine = 0;
+  for (uint32_t i = first; i < last; ++i) mine += chosen(own_keys[i], c * ck + i) ? 1u : 0u;
+  uint32_t packed_total;  // both counts below 2^16: the entries fit the registers
+  const uint32_t packed = block_excl_scan<kSelWaves>((before << 16) | mine, sh.wsum[0], packed_total);
+  uint32_t slot = (packed_total >> 16) + (packed & 0xffffu);
+  int64_t* oidx = a.out_idx + (size_t)row * kk;
+  float* oval = a.out_val ? a.out_val + (size_t)row * kk : nullptr;
+  const uint32_t* own_list = reinterpret_cast<const uint32_t*>(a.lists + (size_t)row * (uint32_t)a.length + c * ck);
+  const uint32_t own_room = min(ck, (uint32_t)a.length - c * ck);
+  for (uint32_t i = first; i < last && mine; ++i) {
+    const uint32_t key = own_keys[i];
+    if (chosen(key, c * ck + i)) {
+      if (slot < kk) {  // always true for consistent counts; keeps writes in the row
+        oidx[slot] = (int64_t)(per == 1u ? own_pos : own_list[own_room + i]);
+        if (oval) oval[slot] = ordered_to_float(key);
+      }
+      ++slot;
+      --mine;
+    }
+  }
+  if (c == 0) {
+    for (uint32_t i = min((uint32_t)a.length, kk) + tid; i < kk; i += kSelThreads) {
+      oidx[i] = -1;
+      if (oval) oval[i] = -__builtin_inff();
+    }
+  }
+  return true;
+}
+
+// The row's counts: the sum of its chunks' (bits 0-30), and how many chunks
+// flagged (bit 31).
+__device__ __forceinline__ void sum_count_parts(const ListArgs& a, uint32_t row, uint32_t chunks) {
+  const uint32_t lane = lane_id();
+  uint32_t sum = 0;
+  uint32_t flags = 0;
+  for (uint32_t j = lane; j < chunks; j += kWave) {
+    const uint32_t part = a.count_parts[(size_t)row * chunks + j];
+    sum += part & 0x7fffffffu;
+    flags += part >> 31;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += (uint32_t)__shfl_xor((int)sum, off, kWave);
+    flags += (uint32_t)__shfl_xor((int)flags, off, kWave);
+  }
+  if (lane == 0) {
+    a.count_out[row] = (int32_t)sum;
+    if (a.flag_out) a.flag_out[row] = (int32_t)flags;
+  }
+}
+
 __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   __shared__ ListShared sh;
-  args_in_sgprs(a.scores, a.lists, a.meta, a.length, a.chunks, a.chunk_keys, a.k, a.total_wgs, a.out_idx,
-                a.out_val);
+  args_in_sgprs(a.scores, a.lists, a.meta, a.length, a.chunks, a.chunk_keys, a.k, a.loads, a.total_wgs,
+                a.out_idx, a.out_val);
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = lane_id();
   const uint32_t wave = tid / kWave;
@@ -487,47 +685,37 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   const float* srow = a.scores + (size_t)row * n;
   const uint64_t* lrow = a.lists + (size_t)row * n;
   DSA_TRACE_MARK(g_trace_select, blockIdx.x, 0);
-  if (a.count_parts && c == 0 && wave == 0) {
-    uint32_t sum = 0;
-    uint32_t flags = 0;
-    for (uint32_t j = lane; j < chunks; j += kWave) {
-      const uint32_t part = a.count_parts[(size_t)row * chunks + j];
-      sum += part & 0x7fffffffu;
-      flags += part >> 31;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      sum += (uint32_t)__shfl_xor((int)sum, off, kWave);
-      flags += (uint32_t)__shfl_xor((int)flags, off, kWave);
-    }
-    if (lane == 0) {
-      a.count_out[row] = (int32_t)sum;
-      if (a.flag_out) a.flag_out[row] = (int32_t)flags;
-    }
-  }
-
   // This thread's list j and its place r among the list's threads.
   const uint32_t tpl = chunks >= (uint32_t)kSelThreads ? 1u : (uint32_t)kSelThreads / chunks;
   const uint32_t j = tid / tpl;
   const uint32_t r = tid % tpl;
   const bool has_list = j < chunks;
   const uint32_t chunk_len = has_list ? min(ck, n - j * ck) : 0u;
-  uint32_t list_len = 0;
-  uint32_t list_bin = 0;
-  uint64_t pre[kListSpec] = {};
-  if (has_list) {
-    const uint32_t* m = a.meta + 2 * ((size_t)row * kMaxListChunks + j);
-    list_len = min(m[0], chunk_len);  // (keeps every read inside the row whatever the workspace holds)
-    list_bin = m[1];
+  uint4 pre[kListVecs];
+  const uint32_t* lwords = reinterpret_cast<const uint32_t*>(lrow + (has_list ? j : 0u) * ck);
+  const BufferRsrc words = make_buffer(lrow, 8u * n);
+  const uint32_t lbase = 2u * (has_list ? j : 0u) * ck;
+  const uint32_t own_room = min(ck, n - c * ck);
+  const uint32_t* own_words = reinterpret_cast<const uint32_t*>(lrow + c * ck);
+  const uint32_t own_pos = tid < own_room ? own_words[own_room + tid] : 0u;
+  const uint2 m = buffer_load_8(make_buffer(a.meta + 2 * (size_t)row * kMaxListChunks, 8u * kMaxListChunks),
+                                has_list ? 8u * j : kPastBuffer);
 #pragma unroll
-    for (int q = 0; q < kListSpec; ++q) {
-      const uint32_t s = r + tpl * q;
-      pre[q] = s < chunk_len ? lrow[j * ck + s] : 0u;
-    }
+  for (int q = 0; q < kListVecs; ++q)
+    pre[q] = load_scores(words, lbase, 4u * (r + tpl * q), q < a.loads ? chunk_len : 0u);
+  const uint32_t list_len = min(m.x, chunk_len);  // (keeps every read inside the row whatever the workspace holds)
+  const uint32_t list_bin = m.y;
+  if (select_lists_fast(a, sh, words, lbase, pre, list_len, list_bin, own_pos, j, r, tpl, row, c)) {
+    if (a.count_parts && c == 0 && wave == 0) sum_count_parts(a, row, chunks);
+    DSA_TRACE_MARK(g_trace_select, blockIdx.x, 4);
+    return;
   }
+  if (a.count_parts && c == 0 && wave == 0) sum_count_parts(a, row, chunks);
+  __syncthreads();  // the shared arrays are taken over below
   bool raw = false;
   auto load_entry = [&](uint32_t s) -> uint64_t {  // entry s of this thread's source
     const uint32_t pos = j * ck + s;
-    return raw ? select_composite(float_to_ordered(srow[pos]), pos) : lrow[pos];
+    return select_composite(raw ? float_to_ordered(srow[pos]) : lwords[s], pos);
   };
 
   uint32_t entries = 0;
@@ -557,12 +745,7 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
       __hip_atomic_fetch_add(&sh.hist[(uint32_t)(x >> 52)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (staged) sh.stage[src_base + s] = x;
     };
-    if (!raw) {
-#pragma unroll
-      for (int q = 0; q < kListSpec; ++q)
-        if (r + tpl * q < src_len) take(r + tpl * q, pre[q]);
-    }
-    for (uint32_t s = r + (raw ? 0u : tpl * kListSpec); s < src_len; s += tpl) take(s, load_entry(s));
+    for (uint32_t s = r; s < src_len; s += tpl) take(s, load_entry(s));
     __syncthreads();
     if (wave == 0) {
       const Locate t = wave_locate<kSelectBins / kWave>(sh.hist, kk, true);
@@ -586,9 +769,6 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   DSA_TRACE_MARK(g_trace_select, blockIdx.x, 1);
   const uint32_t bin = sh.bin;
   auto raw_of = [&](uint32_t list) { return sh.raw[list] != 0u; };
-  auto entry_of = [&](uint32_t s) -> uint64_t {  // entry s of this thread's source
-    return staged ? sh.stage[src_base + s] : load_entry(s);
-  };
   // Entries of the sources before this chunk's: those above the cut's bin
   // are chosen; those inside it are compacted with the rest of the bin.
   // (With at most k entries, every entry of the earlier sources is chosen.)
@@ -607,38 +787,19 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
     before = 0;
     for (uint32_t i = tid; i < sh.base[c]; i += kSelThreads) before += sh.stage[i] >= cstar ? 1u : 0u;
   } else if (bin != kNoBin) {
-    // Entries read in place (raw rounds past the stage): count, scan, then
-    // place the entries of the cut's bin, from the registers that fetched
-    // them where they still hold them, else from memory.
-    const bool in_regs = !raw;
-    const uint32_t spec_end = in_regs ? min(src_len, tpl * kListSpec) : 0u;
+    // Entries read in place (more than the stage holds): count, scan, then
+    // place the entries of the cut's bin.
     uint32_t n_cand = 0;
-#pragma unroll
-    for (int q = 0; q < kListSpec; ++q) {
-      const uint32_t s = r + tpl * q;
-      const uint32_t b = (uint32_t)(pre[q] >> 52);
-      n_cand += (s < spec_end && b == bin) ? 1u : 0u;
-      before += (s < spec_end && b > bin && j < c) ? 1u : 0u;
-    }
-    const uint32_t tail0 = in_regs ? r + tpl * kListSpec : r;
-    for (uint32_t s = tail0; s < src_len; s += tpl) {
-      const uint32_t b = (uint32_t)(entry_of(s) >> 52);
+    for (uint32_t s = r; s < src_len; s += tpl) {
+      const uint32_t b = (uint32_t)(load_entry(s) >> 52);
       n_cand += b == bin ? 1u : 0u;
       before += (b > bin && j < c) ? 1u : 0u;
     }
     uint32_t crowd_total;
     uint32_t slot = block_excl_scan<kSelWaves>(n_cand, sh.wsum[0], crowd_total);
     if (n_cand) {
-#pragma unroll
-      for (int q = 0; q < kListSpec; ++q) {
-        const uint32_t s = r + tpl * q;
-        if (s < spec_end && (uint32_t)(pre[q] >> 52) == bin) {
-          if (slot < (uint32_t)kCandCapacity) sh.cands[slot] = pre[q];
-          ++slot;
-        }
-      }
-      for (uint32_t s = tail0; s < src_len; s += tpl) {
-        const uint64_t x = entry_of(s);
+      for (uint32_t s = r; s < src_len; s += tpl) {
+        const uint64_t x = load_entry(s);
         if ((uint32_t)(x >> 52) == bin) {
           if (slot < (uint32_t)kCandCapacity) sh.cands[slot] = x;
           ++slot;
@@ -669,8 +830,10 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
           const uint32_t mid = (lo + hi + 1) >> 1;
           if (sh.base[mid] <= i) lo = mid; else hi = mid - 1;
         }
-        const uint32_t pos = lo * ck + (i - sh.base[lo]);
-        return raw_of(lo) ? select_composite(float_to_ordered(srow[pos]), pos) : lrow[pos];
+        const uint32_t s = i - sh.base[lo];
+        const uint32_t pos = lo * ck + s;
+        const uint32_t* words = reinterpret_cast<const uint32_t*>(lrow + lo * ck);
+        return select_composite(raw_of(lo) ? float_to_ordered(srow[pos]) : words[s], pos);
       };
       cstar = radix_cut<true>(bin, sh.want, entries, entry_at, digits, sh.radix);
       before = 0;
@@ -688,7 +851,7 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   auto own_at = [&](uint32_t s) -> uint64_t {
     if (staged) return sh.stage[own0 + s];
     const uint32_t pos = c * ck + s;
-    return raw_of(c) ? select_composite(float_to_ordered(srow[pos]), pos) : lrow[pos];
+    return select_composite(raw_of(c) ? float_to_ordered(srow[pos]) : own_words[s], pos);
   };
   uint32_t mine = 0;
   for (uint32_t i = first; i < last; ++i) mine += own_at(i) >= cstar ? 1u : 0u;
@@ -709,7 +872,7 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
     const uint64_t x = own_at(i);
     if (x >= cstar) {
       if (slot < kk) {  // always true for consistent counts; keeps writes in the row
-        oidx[slot] = (int64_t)(~(uint32_t)x);
+        oidx[slot] = (int64_t)(raw_of(c) ? c * ck + i : own_words[own_room + i]);
         if (oval) oval[slot] = ordered_to_float((uint32_t)(x >> 32));
       }
       ++slot;
@@ -825,6 +988,11 @@ int launch_select_lists(const float* scores, int64_t rows, int64_t length, int64
   a.chunks = plan.chunks;
   a.chunk_keys = plan.chunk_keys;
   a.k = (int32_t)k;
+  const int64_t per_load = 4 * (plan.chunks >= kSelThreads ? 1 : kSelThreads / plan.chunks);  // entries of a list
+  const int64_t expected = 2 * (int64_t)plan.quota + 8;
+  const int64_t most = expected < plan.chunk_keys ? expected : plan.chunk_keys;
+  const int64_t loads = (most + per_load - 1) / per_load;
+  a.loads = (int32_t)(loads < kListVecs ? loads : kListVecs);
   a.total_wgs = (uint32_t)(rows * plan.chunks);
   a.out_idx = out_idx;
   a.out_val = out_val;

@@ -21,7 +21,7 @@ struct SelectWorkspace {
   uint32_t* meta;        // [rows][4]: threshold bin, rank inside it, valid count
   uint32_t* above;       // [rows][chunks]: per-chunk count above the bin
   uint64_t* cand;        // [rows][length]: chunk j's candidates at [j * kSelectChunk, ...)
-                         // (candidate lists: list j at [j * chunk_keys, ...))
+                         // (candidate lists: list j at [j * chunk_keys, ...), scores, then positions)
   uint32_t* list_meta;   // [rows][kMaxListChunks][2]: list length, lowest 12-bit bin listed
   int64_t bytes;
 };

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void temporal_static_kernel(Tempo
   DSA_TRACE_MARK(g_trace_static, blockIdx.x, 5);
   // 5. The chunk's candidate list for the list select.
   write_chunk_list<kFusedWaves>(hist, chunk_scores, p.chunk_keys, n_chunk, base, p.quota,
-                                a.ws.select.cand + (size_t)row * L + base,
+                                reinterpret_cast<uint32_t*>(a.ws.select.cand + (size_t)row * L + base), n_chunk,
                                 a.ws.select.list_meta + 2 * ((size_t)row * kMaxListChunks + c), &s_list_bin, s_wsum);
   DSA_TRACE_MARK(g_trace_static, blockIdx.x, 6);
 }

@@ -477,17 +477,6 @@ struct RowShared {
   uint64_t cstar;
 };
 
-// Inclusive scans of 64 lanes by DPP for the minimum and maximum; the value
-// of the whole wave is read off the four row ends.
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x111, 0xf, 0xf, false));
-  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x112, 0xf, 0xf, false));
-  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x114, 0xf, 0xf, false));
-  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x118, 0xf, 0xf, false));
-  return min(min((uint32_t)__builtin_amdgcn_readlane(x, 15), (uint32_t)__builtin_amdgcn_readlane(x, 31)),
-             min((uint32_t)__builtin_amdgcn_readlane(x, 47), (uint32_t)__builtin_amdgcn_readlane(x, 63)));
-}
-
 // Shift that brings keys up to `span` above their origin into kRowBins bins.
 __device__ __forceinline__ int bin_shift(uint32_t span) { return max(0, 20 - (int)__clz((int)(span | 1u))); }
 
@@ -554,7 +543,7 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
       hi = max(hi, key[e]);
     }
     lo = wave_min_u32(lo);
-    hi = ~wave_min_u32(~hi);
+    hi = wave_max_u32(hi);
     if (lane == 0) {
       sh.wave_lo[wave] = lo;
       sh.wave_hi[wave] = hi;

@@ -33,6 +33,18 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
   return x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
 }
 
+// Minimum (and, of the complement, maximum) over the 64 lanes: DPP row shifts,
+// then the four row ends, uniform over the wave.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x111, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x112, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x114, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x118, 0xf, 0xf, false));
+  return min(min((uint32_t)__builtin_amdgcn_readlane(x, 15), (uint32_t)__builtin_amdgcn_readlane(x, 31)),
+             min((uint32_t)__builtin_amdgcn_readlane(x, 47), (uint32_t)__builtin_amdgcn_readlane(x, 63)));
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) { return ~wave_min_u32(~x); }
+
 // Exclusive scan over the workgroup: one barrier; `ws` (16 words) must not be
 // rewritten until every thread has passed a later barrier.
 template <int kWaves>
