@@ -382,12 +382,19 @@ __global__ __launch_bounds__(kRoundThreads) void temporal_round_kernel(TemporalA
 // decided by bins alone, one inside it needs the exact k-th largest, a select
 // among the cut bin's joined keys.
 // ---------------------------------------------------------------------------
-constexpr int kResolveThreads = 512;
+// The replay's code runs once or a few times per launch, so what bounds it
+// outside wave 0's chain is fetching its instructions as much as memory: two
+// keys a thread in registers over 1024 threads, the rest read again in rolled
+// loops.  512 threads that read every key from memory in batches of four ->
+// this, a 4 x 16639 step with k 2048, MI355X: 88.6 -> 84.3 us; 10993 keys, k
+// 256: 98.1 -> 97.4 (with four keys a thread 83.8 and 99.5 to 100.6; 512
+// threads and eight keys a thread 88.6 and 101.7).
+constexpr int kResolveThreads = 1024;
 constexpr int kResolveWaves = kResolveThreads / kWave;
 constexpr int kSortCap = 8192;  // keys the replay sorts in LDS (more: in the workspace)
 constexpr int kBins = 4096;
 constexpr int kCutDigits = 1024;  // 10-bit digits of the select inside the cut bin
-constexpr int kKeyBatch = 8;      // key values per thread in flight in the replay's first read
+constexpr int kKeyBatch = 2;      // keys per thread in the replay's first read, kept in registers
 
 struct ResolveShared {
   uint32_t val[kSortCap];   // ordered keys, by bin
@@ -465,8 +472,51 @@ __device__ __forceinline__ uint32_t cut_select(P32 val, P8 join, uint32_t s0, ui
   return base + (hi << lo_bits);
 }
 
+// The round's keys of one row: place i < k is the i-th of the running k
+// largest, the others the listed keys.  A key is its ordered value and a high
+// word: the running key's index, or a listed entry's group << 17 | index.
+struct KeySource {
+  const uint32_t* run;
+  const uint32_t* idx;
+  const uint64_t* list;
+  uint32_t k;
+  uint32_t last;  // the last list entry that may be read
+
+  __device__ __forceinline__ KeySource(const TemporalArgs& a, const RoundPlan& rp, int row, uint32_t n_listed)
+      : run(a.ws.run + run_offset(a, rp.round, row)),
+        idx(a.ws.run_idx + run_offset(a, rp.round, row)),
+        list(a.ws.entries + (size_t)row * a.ws.list_capacity),
+        k((uint32_t)a.k),
+        last(n_listed ? n_listed - 1u : 0u) {}
+  __device__ __forceinline__ uint2 at(uint32_t i) const {
+    const uint32_t* entry = reinterpret_cast<const uint32_t*>(list + min(i - k, last));  // (wraps below k: clamped)
+    const uint32_t* low = i < k ? run + i : entry;
+    const uint32_t* high = i < k ? idx + i : entry + 1;
+    return make_uint2(*low, *high);
+  }
+};
+
+// Adds one to counts[at] for every active lane and returns the lane's place
+// among them: one atomic for the wave when all lanes name the same count, as
+// listed keys, stored by tile, mostly do (64 lanes on one address take 64
+// turns).
+__device__ __forceinline__ uint32_t wave_count(uint32_t* counts, uint32_t at) {
+  const uint64_t active = __ballot(true);
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+  if (__ballot(at == first) == active) {
+    const uint32_t below = lanes_below(active);
+    uint32_t base = 0u;
+    if (below == 0u)
+      base = __hip_atomic_fetch_add(&counts[first], (uint32_t)__builtin_popcountll(active), __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + below;
+  }
+  return __hip_atomic_fetch_add(&counts[at], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 template <bool kSpill>
 __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPlan& rp, ResolveShared& sh,
+                                            const uint32_t (&kv)[kKeyBatch], const uint32_t (&kh)[kKeyBatch],
                                             uint32_t n_listed, uint32_t max_key, uint32_t floor_key,
                                             uint32_t seed_tau, uint64_t t_start) {
   const int tid = threadIdx.x;
@@ -485,15 +535,21 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
   uint32_t* val = kSpill ? a.ws.spill_val + spill_at : sh.val;
   uint32_t* item = kSpill ? a.ws.spill_item + spill_at : sh.item;
   uint8_t* join = kSpill ? a.ws.spill_join + spill_at : sh.join;
-  const uint32_t* run = a.ws.run + run_offset(a, rp.round, row);
-  const uint64_t* list = a.ws.entries + (size_t)row * a.ws.list_capacity;
-  auto each_run = [&](auto f) {
-    batched<4>((uint32_t)tid, (uint32_t)k, kResolveThreads, [&](uint32_t i) { return run[i]; },
-               [&](uint32_t, uint32_t v) { f(v); });
-  };
-  auto each_listed = [&](auto f) {
-    batched<4>((uint32_t)tid, n_listed, kResolveThreads, [&](uint32_t e) { return list[e]; },
-               [&](uint32_t, uint64_t x) { f(x); });
+  const uint32_t n_keys = (uint32_t)k + n_listed;
+  // f(key's place, value, high word) for this thread's keys: the first
+  // kKeyBatch from the registers that fetched them, the rest from memory.
+  auto each_key = [&](auto f) {
+#pragma unroll
+    for (int j = 0; j < kKeyBatch; ++j)
+      if ((uint32_t)(tid + j * kResolveThreads) < n_keys) f((uint32_t)(tid + j * kResolveThreads), kv[j], kh[j]);
+    if (n_keys > (uint32_t)(kKeyBatch * kResolveThreads)) {
+      const KeySource keys(a, rp, row, n_listed);
+#pragma unroll 1
+      for (uint32_t i = (uint32_t)(tid + kKeyBatch * kResolveThreads); i < n_keys; i += kResolveThreads) {
+        const uint2 x = keys.at(i);
+        f(i, x.x, x.y);
+      }
+    }
   };
 
   // Bin and group counts (E counts the joined keys: run's).
@@ -508,19 +564,18 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
   }
   __syncthreads();
   uint32_t above = 0;
-  each_run([&](uint32_t v) {
+  each_key([&](uint32_t i, uint32_t v, uint32_t high) {
     const uint32_t b = (v - floor_key) >> shift;
     __hip_atomic_fetch_add(&sh.end[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_add(&sh.E[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    above += b > 0 ? 1u : 0u;
+    if (i < (uint32_t)k) {
+      __hip_atomic_fetch_add(&sh.E[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      above += b > 0 ? 1u : 0u;
+    } else {
+      wave_count(sh.gend, (high >> 17) - (uint32_t)g_begin);
+    }
   });
   for (int off = 32; off > 0; off >>= 1) above += (uint32_t)__shfl_xor((int)above, off, kWave);
   if (lane == 0 && above) __hip_atomic_fetch_add(&sh.above, above, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  each_listed([&](uint64_t x) {
-    const uint32_t b = ((uint32_t)x - floor_key) >> shift;
-    __hip_atomic_fetch_add(&sh.end[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_add(&sh.gend[(int)(x >> 49) - g_begin], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  });
   __syncthreads();
   // Exclusive scans: end[b] <- first slot of bin b, gend[g] <- first item of
   // group g (the scatter's cursors; past it they hold each one's end).
@@ -578,22 +633,16 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
   }
   __syncthreads();
   // Scatter: run's keys joined, listed keys not yet; listed keys' items by group.
-  each_run([&](uint32_t v) {
+  each_key([&](uint32_t i, uint32_t v, uint32_t high) {
     const uint32_t slot = __hip_atomic_fetch_add(&sh.end[(v - floor_key) >> shift], 1u, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_WORKGROUP);
     val[slot] = v;
-    join[slot] = 1;
-  });
-  each_listed([&](uint64_t x) {
-    const uint32_t v = (uint32_t)x;
-    const uint32_t slot = __hip_atomic_fetch_add(&sh.end[(v - floor_key) >> shift], 1u, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
-    val[slot] = v;
-    join[slot] = 0;
-    const uint32_t blk = (uint32_t)((x >> 32) & 0x1ffffu) / (uint32_t)a.block_size;
-    const uint32_t at = __hip_atomic_fetch_add(&sh.gend[(int)(x >> 49) - g_begin], 1u, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-    item[at] = slot | (blk << 18);
+    join[slot] = i < (uint32_t)k ? 1 : 0;
+    if (i >= (uint32_t)k) {
+      const uint32_t blk = (high & 0x1ffffu) / (uint32_t)a.block_size;
+      const uint32_t at = wave_count(sh.gend, (high >> 17) - (uint32_t)g_begin);
+      item[at] = slot | (blk << 18);
+    }
   });
   __syncthreads();
 
@@ -717,10 +766,7 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
           const uint32_t t = exact_tau();
           if (verdict == 2) verdict = prunes(uk, t) ? 0 : 1;
         }
-        if (active) {
-          a.evaluated[(size_t)row * nb + blk] = (uint8_t)verdict;
-          sh.kept[blk] = (uint8_t)verdict;
-        }
+        if (active) sh.kept[blk] = (uint8_t)verdict;
         const bool reset = active && verdict == 0 && !prunes(uk, floor_key);
         const uint64_t m = __ballot(reset);
         if (reset) sh.resets[nreset + lanes_below(m)] = (uint16_t)blk;
@@ -838,17 +884,23 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
 #ifdef DSA_PHASE_TRACE
   const uint64_t t_tail0 = wall_clock64();
 #endif
-  // After the loop the LDS key arrays are free: sh.item and sh.val serve as
-  // staging (in the spill case they were never used).
+  // The round's decisions (stored here by every thread: a store per step of
+  // the loop is left out of wave 0's chain).
+  for (int i = tid; i < n_pos; i += kResolveThreads) {
+    const uint32_t blk = sh.blk[i];
+    a.evaluated[(size_t)row * nb + blk] = sh.kept[blk];
+  }
+  // After the loop the LDS key arrays are free: sh.item serves as staging (in
+  // the spill case it was never used).
   const int bs = a.block_size;
   const int L = a.length;
   const uint32_t t = sh.tau;
-  const size_t run_at = run_offset(a, rp.round, row);
-  const uint32_t* run_in = a.ws.run + run_at;
-  const uint32_t* idx_in = a.ws.run_idx + run_at;
   // A listed key joined iff its block was kept (every listed key's block was
   // decided by this round).
-  auto listed_joined = [&](uint64_t x) { return sh.kept[((uint32_t)(x >> 32) & 0x1ffffu) / (uint32_t)bs] != 0; };
+  auto joined = [&](uint32_t i, uint32_t high) {
+    return i < (uint32_t)k || sh.kept[(high & 0x1ffffu) / (uint32_t)bs] != 0;
+  };
+  auto index_of = [&](uint32_t i, uint32_t high) { return i < (uint32_t)k ? high : high & 0x1ffffu; };
   if (!rp.last_round) {
     // The next round starts from the exact k largest, each with its key: the
     // joined keys above the threshold (the run's and the listed ones), then
@@ -856,17 +908,13 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
     const size_t out_at = run_offset(a, rp.round + 1, row);
     uint32_t* run_out = a.ws.run + out_at;
     uint32_t* idx_out = a.ws.run_idx + out_at;
-    auto emit = [&](uint32_t v, uint32_t key) {
-      const uint32_t j = __hip_atomic_fetch_add(&sh.n_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      run_out[j] = v;
-      idx_out[j] = key;
-    };
-    for (int i = tid; i < k; i += kResolveThreads)
-      if (run_in[i] > t) emit(run_in[i], idx_in[i]);
-    for (uint32_t e = (uint32_t)tid; e < n_listed; e += kResolveThreads) {
-      const uint64_t x = list[e];
-      if ((uint32_t)x > t && listed_joined(x)) emit((uint32_t)x, (uint32_t)(x >> 32) & 0x1ffffu);
-    }
+    each_key([&](uint32_t i, uint32_t v, uint32_t high) {
+      if (v > t && joined(i, high)) {
+        const uint32_t j = __hip_atomic_fetch_add(&sh.n_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        run_out[j] = v;
+        idx_out[j] = index_of(i, high);
+      }
+    });
     __syncthreads();
     for (uint32_t c = sh.n_out + (uint32_t)tid; c < (uint32_t)k; c += kResolveThreads) {
       run_out[c] = t;
@@ -898,12 +946,9 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
         else chosen += 1u << 20;  // no index: not this path
       };
-      for (int i = tid; i < k; i += kResolveThreads)
-        if (run_in[i] >= t) mark(idx_in[i]);
-      for (uint32_t e = (uint32_t)tid; e < n_listed; e += kResolveThreads) {
-        const uint64_t x = list[e];
-        if ((uint32_t)x >= t && listed_joined(x)) mark((uint32_t)(x >> 32) & 0x1ffffu);
-      }
+      each_key([&](uint32_t i, uint32_t v, uint32_t high) {
+        if (v >= t && joined(i, high)) mark(index_of(i, high));
+      });
       uint32_t total;
       block_excl_scan<kResolveWaves>(chosen, sh.wsum, total);  // its barrier also ends the marking
       if (total == (uint32_t)k) {
@@ -931,6 +976,7 @@ __device__ __forceinline__ void resolve_row(const TemporalArgs& a, const RoundPl
     }
     if (finished || a.replay_qk) {
       // Keys scored: the seeds and every key of a kept block, each once.
+      __syncthreads();  // every decision of the round is stored
       const int nb = a.blocks;
       const uint32_t* mask = a.ws.seed_mask + (size_t)row * words;
       uint32_t scored = 0u;
@@ -1007,14 +1053,11 @@ __global__ __launch_bounds__(kResolveThreads) void temporal_resolve_kernel(Tempo
   const int wave = tid >> 6;
   const uint32_t* order = a.ws.order + (size_t)row * nb + rp.pos_begin;
   const double* upper = a.ws.upper_pos + (size_t)row * nb + rp.pos_begin;
-  const uint32_t* run = a.ws.run + run_offset(a, rp.round, row);
-  const uint64_t* list = a.ws.entries + (size_t)row * a.ws.list_capacity;
   // The setup's inputs are read in one round trip: the positions' blocks and
-  // bounds (at most four per thread), the list's length, the floor, the
-  // seeds' threshold, and the first kKeyBatch key values per thread, each
-  // from the running k largest or the list (one dword: an entry's value is
-  // its low word), list reads clamped to its capacity until its length is
-  // known.
+  // bounds (at most two per thread), the list's length, the floor, the
+  // seeds' threshold, and the first kKeyBatch keys per thread, each from the
+  // running k largest or the list, list reads clamped to its capacity until
+  // its length is known.  These keys stay in registers.
   const uint32_t n_listed = a.ws.list_total[(size_t)row * kMaxRounds + rp.round];
   const uint32_t floor_key = a.ws.floor[row];
   const uint32_t seed_tau = a.ws.tau[row];
@@ -1027,15 +1070,16 @@ __global__ __launch_bounds__(kResolveThreads) void temporal_resolve_kernel(Tempo
     pb[j] = order[i];
     pu[j] = upper[i];
   }
-  const uint32_t cap_last = (uint32_t)a.ws.list_capacity - 1u;
-  auto key_value = [&](uint32_t i, uint32_t last) {
-    const uint32_t e = min(i - (uint32_t)k, last);  // (wraps below k: clamped, unused)
-    const uint32_t* p = i < (uint32_t)k ? run + i : reinterpret_cast<const uint32_t*>(list + e);
-    return *p;
-  };
-  uint32_t kv[kKeyBatch];
+  uint32_t kv[kKeyBatch], kh[kKeyBatch];
+  {
+    const KeySource keys(a, rp, row, (uint32_t)a.ws.list_capacity);
 #pragma unroll
-  for (int j = 0; j < kKeyBatch; ++j) kv[j] = key_value((uint32_t)(tid + j * kResolveThreads), cap_last);
+    for (int j = 0; j < kKeyBatch; ++j) {
+      const uint2 x = keys.at((uint32_t)(tid + j * kResolveThreads));
+      kv[j] = x.x;
+      kh[j] = x.y;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < kPosPer; ++j) {
     const int i = tid + j * kResolveThreads;
@@ -1050,14 +1094,9 @@ __global__ __launch_bounds__(kResolveThreads) void temporal_resolve_kernel(Tempo
 #pragma unroll
   for (int j = 0; j < kKeyBatch; ++j)
     if ((uint32_t)(tid + j * kResolveThreads) < n_keys) mx = max(mx, kv[j]);
-  const uint32_t list_last = n_listed ? n_listed - 1u : 0u;
-  for (uint32_t i0 = (uint32_t)tid + kKeyBatch * kResolveThreads; i0 < n_keys; i0 += kKeyBatch * kResolveThreads) {
-#pragma unroll
-    for (int j = 0; j < kKeyBatch; ++j) kv[j] = key_value(i0 + (uint32_t)(j * kResolveThreads), list_last);
-#pragma unroll
-    for (int j = 0; j < kKeyBatch; ++j)
-      if (i0 + (uint32_t)(j * kResolveThreads) < n_keys) mx = max(mx, kv[j]);
-  }
+  const KeySource keys(a, rp, row, n_listed);
+  batched<kKeyBatch>((uint32_t)(tid + kKeyBatch * kResolveThreads), n_keys, kResolveThreads,
+                     [&](uint32_t i) { return keys.at(i).x; }, [&](uint32_t, uint32_t v) { mx = max(mx, v); });
   for (int off = 32; off > 0; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, kWave));
   if (lane == 0) sh.wsum[wave] = mx;
   __syncthreads();
@@ -1065,9 +1104,9 @@ __global__ __launch_bounds__(kResolveThreads) void temporal_resolve_kernel(Tempo
 #pragma unroll
   for (int w = 0; w < kResolveWaves; ++w) max_key = max(max_key, sh.wsum[w]);
   if (n_keys <= (uint32_t)kSortCap)
-    resolve_row<false>(a, rp, sh, n_listed, max_key, floor_key, seed_tau, t_start);
+    resolve_row<false>(a, rp, sh, kv, kh, n_listed, max_key, floor_key, seed_tau, t_start);
   else
-    resolve_row<true>(a, rp, sh, n_listed, max_key, floor_key, seed_tau, t_start);
+    resolve_row<true>(a, rp, sh, kv, kh, n_listed, max_key, floor_key, seed_tau, t_start);
 }
 
 // Round splits, as fractions of the scan's groups: DSA_AMD_TEMPORAL_ROUNDS, a
