@@ -502,7 +502,10 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
   const int64_t out_base = v * (int64_t)k;
 
   // Element e of a thread is position kStep (e / 4) + 4 tid + e % 4; its order
-  // key, 0 past the row (the loads return 0 there).
+  // key, 0 past the row (the loads return 0 there).  One bit pattern in the row
+  // has key 0 as well, the NaN 0xffffffff: such an element is no candidate, as
+  // in topk_kernel, so a row may hold fewer than k keys also where n > k, and
+  // the output is padded from the number of keys found.
   uint32_t key[EPT];
   auto pos_of = [&](int e) { return kStep * (e >> 2) + 4 * tid + (e & 3); };
   {
@@ -527,14 +530,15 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
 
   bool done = false;  // sorted output written
   if (n <= k) {
-    // Every element is chosen.
+    // Every element with a key is chosen.
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < EPT; e += 4)
-      if (pos_of(e) < n) {
-        const int left = min(4, n - pos_of(e));
-        atomicOr(&sh.bits[pos_of(e) >> 5], ((1u << left) - 1u) << (pos_of(e) & 31));
-      }
+    for (int e = 0; e < EPT; e += 4) {
+      uint32_t set = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) set |= key[e + i] != 0 ? 1u << i : 0u;
+      if (set) atomicOr(&sh.bits[pos_of(e) >> 5], set << (pos_of(e) & 31));
+    }
   } else {
     uint32_t lo = 0xffffffffu, hi = 0u;
 #pragma unroll
@@ -724,7 +728,8 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
     }
     if (!resolved) {
       // Radix select of the k-th key over the whole row (12, 12 and 8 bits),
-      // then the ties at it in index order.
+      // then the ties at it in index order.  With fewer than k keys in the row
+      // there is no k-th (the first pass finds no bin): prefix 0, every key.
       uint32_t prefix = 0, prefix_mask = 0, want = (uint32_t)k;
 #pragma unroll 1
       for (int pass = 0; pass < 3; ++pass) {
@@ -745,6 +750,10 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
           }
         }
         __syncthreads();
+        if (sh.digit == kNoBin) {
+          want = 0;
+          break;
+        }
         prefix |= sh.digit << sft;
         prefix_mask |= dmask << sft;
         want = sh.rem;
@@ -773,13 +782,14 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
       sh.bits[tid] |= chosen;
     }
   }
-  const int chosen_n = min(n, k);
+  int chosen_n = k;  // (a sorted output is written by then only with k candidates)
   if (!done) {
     __syncthreads();
     uint32_t word = sh.bits[tid];
     uint32_t total;
     uint32_t p = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[1], total);
-    // Exactly chosen_n bits are set; the bound only guards the buffers.
+    // min(keys in the row, k) bits are set; the bound only guards the buffers.
+    chosen_n = min((int)total, k);
     while (word) {
       const uint32_t at = 32u * tid + (uint32_t)__builtin_ctz(word);
       word &= word - 1;
@@ -805,7 +815,7 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
       }
     }
   }
-  // Padding when the row has fewer than k elements.
+  // Padding when the row has fewer than k keys.
   for (int i = chosen_n + tid; i < k; i += kTopkThreads) {
     if (a.out_idx) a.out_idx[out_base + i] = -1;
     if (a.out_val) a.out_val[out_base + i] = -__builtin_inff();

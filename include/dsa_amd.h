@@ -231,7 +231,8 @@ int dsa_promote_blocks(const uint8_t* direct_blocks, const float* block_max,
 /* ------------------------------------------------------------------------
  * Exact top-k per row with the reference's stable_topk semantics
  * (metrics.py:9-22): the k largest values, ties at the cut-off resolved
- * towards the lower index; -0.0 equals +0.0.  NaN is not supported.
+ * towards the lower index; -0.0 equals +0.0.  NaN is not supported
+ * (the pattern 0xffffffff is never chosen, other NaNs rank by their bits).
  *
  *   scores      [rows, row_stride] fp32, the first `length` entries of a row
  *               are candidates

@@ -60,3 +60,34 @@ def test_rows_match_oracle(device, kind, length, k) -> None:
         chosen = want >= 0
         np.testing.assert_array_equal(values[r][chosen].view(np.uint32), host[r][want[chosen]].view(np.uint32))
         assert np.isneginf(values[r][~chosen]).all()
+
+
+@pytest.mark.parametrize("length,k,keys", [
+    (1000, 1000, 999),    # every element with a key, k the row
+    (4100, 4096, 4095),   # one key short of k
+    (4100, 4096, 4096),   # exactly k keys
+    (5000, 2048, 3),      # far fewer, full histogram
+    (20000, 100, 60),     # and a sampled one
+    (32768, 2048, 0),     # a row of poison alone
+    (40000, 300, 7),      # chunks and their merge
+])
+def test_rows_of_all_ones_bits_are_padded(device, length, k, keys) -> None:
+    # The NaN 0xffffffff is the one value without an order key: never chosen,
+    # the output padded with -1 and -inf after the elements that have one.
+    print(f"topk all-ones bits L={length} k={k} keys={keys}", flush=True)
+    rng = np.random.default_rng(length + keys)
+    host = np.full((3, length), 0xFFFFFFFF, dtype=np.uint32).view(np.float32)
+    for r in range(3):
+        host[r, rng.permutation(length)[:keys]] = rng.normal(size=keys).astype(np.float32)
+    x = torch.from_numpy(host).to(device)
+    # (past 32768 elements index order takes the distributed select, which ranks these NaNs last instead)
+    for by_rank in (True, False) if length <= metrics.MAX_ROW else (True,):
+        idx, val = metrics.topk(x, k, sorted=by_rank, return_values=True)
+        idx, val = idx.cpu().numpy(), val.cpu().numpy()
+        for r in range(3):
+            at = np.flatnonzero(~np.isnan(host[r]))
+            order = T.topk_sorted_padded(host[r][at], k, at.size) if by_rank else T.topk_index_order(host[r][at], k, at.size)
+            want = np.where(order >= 0, at[order] if at.size else -1, -1)
+            assert idx[r].tolist() == want.tolist(), (r, by_rank)
+            np.testing.assert_array_equal(val[r][want >= 0], host[r][want[want >= 0]])
+            assert np.isneginf(val[r][want < 0]).all()
