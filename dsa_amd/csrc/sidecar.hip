@@ -353,7 +353,10 @@ extern "C" int dsa_encode_keys_rows(const void* hidden, int64_t hidden_stride, i
       reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(DSA_STATUS_WORKSPACE_TOO_SMALL, "needs dsa_encode_keys_workspace_bytes(tokens, kdim, dim) bytes of "
                                                 "16-byte aligned workspace");
-  if (tokens > 16 && dim == kHeadDim && rope_dim == 64 && out_dtype == kBF16) {
+  // finish_keys_kernel stores 8 bytes at a time; rows that are not 8-byte
+  // aligned take the epilogue, which stores pairs (or rejects odd strides).
+  if (tokens > 16 && dim == kHeadDim && rope_dim == 64 && out_dtype == kBF16 && out_row_stride % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(out) % 8 == 0) {
     DSA_REQUIRE(tokens <= 0x7fffffffLL && kdim > 0 && kdim % 8 == 0, "kdim %lld must be a positive multiple of 8",
                 (long long)kdim);
     DSA_REQUIRE(out_row_stride >= dim, "row strides must cover dim");

@@ -785,8 +785,8 @@ int dsa_encode_queries_epilogue(const void* proj, const float* proj_weights, con
 /* encode_keys (sidecar.py:74-76) of bf16 hidden rows with a bf16 wk [dim][kdim]
  * in one call, with the LayerNorm's weight and bias in ln_dtype
  * (DSA_DTYPE_F32 or DSA_DTYPE_BF16).  More than 16 tokens of 128 dims, 64 of
- * them rotated, with a bf16 out: partial sums of wk over runs of k, then the
- * rows from their sums.  Otherwise dsa_project_rows (at most 16 tokens, kdim a
+ * them rotated, with a bf16 out of 8-byte aligned rows: partial sums of wk over
+ * runs of k, then the rows from their sums.  Otherwise dsa_project_rows (at most 16 tokens, kdim a
  * multiple of 32, dim of 16) or dsa_project_gemm, then
  * dsa_encode_keys_epilogue.  Limits are those calls'; workspace (16-byte
  * aligned) holds dsa_encode_keys_workspace_bytes(tokens, kdim, dim). */

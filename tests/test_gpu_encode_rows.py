@@ -97,6 +97,47 @@ def test_keys_equal_separate_calls(device, tokens, hidden_size, norm_dtype, cach
     assert ((got.double() - wide).abs() <= 2.0**-6 * size + 1e-3 * size.mean()).all()
 
 
+@pytest.mark.parametrize("tokens", [16, 17, 300])
+def test_key_rows_off_an_8_byte_boundary(device, tokens) -> None:
+    # A cache view that starts two elements into its storage, and row strides of
+    # 130 (even, not whole 8-byte steps) and 129 (odd: rejected for any batch).
+    print(f"encode keys misaligned rows tokens={tokens}", flush=True)
+    gen = torch.Generator().manual_seed(23 + tokens)
+    module = sidecar.LightningIndexerSidecar(hidden_size=256).to(device=device, dtype=torch.bfloat16).eval()
+    hidden = torch.randn(tokens, 256, generator=gen).to(device, torch.bfloat16)
+    positions = torch.randint(0, 40000, (tokens,), generator=gen).to(device)
+    rows = torch.randperm(400, generator=gen)[:tokens].to(device)
+    store = torch.zeros(400 * 128 + 2, device=device, dtype=torch.bfloat16)
+    view = store[2:].view(400, 128)
+    module.encode_keys(hidden, positions, out=view, out_rows=rows)
+    # The separate calls' rows, which store two elements at a time.
+    proj = module._project(hidden, module.wk.weight)
+    ln_w, ln_b = module.k_norm.weight.detach().float(), module.k_norm.bias.detach().float()
+    want = torch.zeros(400, 128, device=device, dtype=torch.bfloat16)
+    _lib.call("dsa_encode_keys_epilogue", proj.data_ptr(), _lib.DTYPE_BF16, 128, ln_w.data_ptr(), ln_b.data_ptr(), 1e-6,
+              positions.data_ptr(), 64, 10000.0, want.data_ptr(), _lib.DTYPE_BF16, 128, rows.data_ptr(), 400, tokens, 128,
+              _stream())
+    assert torch.equal(view.view(torch.int16), want.view(torch.int16))
+    assert (store[:2] == 0).all()
+
+    need = int(_lib.query("dsa_encode_keys_workspace_bytes", tokens, 256, 128))
+    ws = torch.empty(need, device=device, dtype=torch.uint8)
+
+    def strided(stride):
+        out = torch.zeros(400 * stride, device=device, dtype=torch.bfloat16)
+        _lib.call("dsa_encode_keys_rows", hidden.data_ptr(), 256, tokens, 256, module.wk.weight.data_ptr(), 128,
+                  ws.data_ptr(), need, module.k_norm.weight.data_ptr(), module.k_norm.bias.data_ptr(), _lib.DTYPE_BF16,
+                  1e-6, positions.data_ptr(), 64, 10000.0, out.data_ptr(), _lib.DTYPE_BF16, stride, rows.data_ptr(), 400,
+                  _stream())
+        return out.view(400, stride)
+
+    got = strided(130)
+    assert torch.equal(got[:, :128].contiguous().view(torch.int16), want.view(torch.int16))
+    assert (got[:, 128:] == 0).all()
+    with pytest.raises(RuntimeError, match="even"):
+        strided(129)
+
+
 @pytest.mark.parametrize("kdim,strided", [(64, False), (136, False), (192, True), (2048, False)])
 def test_wq_tiles_agree(device, kdim, strided) -> None:
     # 1100 tokens x 8192 features: 160 wide tiles (kdim a multiple of 64, one to
