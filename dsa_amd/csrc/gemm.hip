@@ -862,17 +862,30 @@ int32_t narrow_k(int64_t tokens, int64_t kdim) {
   return (int32_t)kper;
 }
 
-int64_t narrow_parts_bytes(int64_t tokens, int64_t kdim, int64_t features) {
+// Tokens whose partial sums one launch leaves: at most kNarrowParts bytes of
+// them, so that the workspace does not grow with the batch (the fp32 wq of
+// 4096 tokens, hidden 2048, would leave 512 MiB, of 65000 tokens 8 GiB); longer
+// batches take a launch per slice.
+constexpr int64_t kNarrowParts = int64_t(64) << 20;
+int64_t narrow_slice(int64_t tokens, int64_t kdim, int64_t features) {
   const int64_t kper = narrow_k(tokens, kdim);
-  return (kdim + kper - 1) / kper * tokens * features * (int64_t)sizeof(float);
+  const int64_t token_bytes = (kdim + kper - 1) / kper * features * (int64_t)sizeof(float);
+  const int64_t most = std::max<int64_t>(kNarrowParts / token_bytes / kNarrowTok, 1) * kNarrowTok;
+  return std::min(tokens, most);
 }
 
-// Partial sums of a narrow product, with the rotation table of `rope` (its
-// table nullable) beside it.
+int64_t narrow_parts_bytes(int64_t tokens, int64_t kdim, int64_t features) {
+  const int64_t kper = narrow_k(tokens, kdim);
+  return (kdim + kper - 1) / kper * narrow_slice(tokens, kdim, features) * features * (int64_t)sizeof(float);
+}
+
+// Partial sums of a narrow product over the slice of a.tokens (of `batch`, from
+// which k's split follows), with the rotation table of `rope` (its table
+// nullable) beside it.
 template <bool kF32>
-int launch_narrow(NarrowArgs& a, const RopeTableArgs& rope, hipStream_t stream) {
+int launch_narrow(NarrowArgs& a, int64_t batch, const RopeTableArgs& rope, hipStream_t stream) {
   constexpr int kFeat = kF32 ? 64 : 128;
-  a.kper = narrow_k(a.tokens, a.kdim);
+  a.kper = narrow_k(batch, a.kdim);
   a.splits = (a.kdim + a.kper - 1) / a.kper;
   const int64_t blocks = (int64_t)a.splits * ((a.features + kFeat - 1) / kFeat) *
                          ((a.tokens + kNarrowTok - 1) / kNarrowTok);
@@ -991,20 +1004,24 @@ static int project_weights(const GemmArgs& a, const float* weight, int64_t featu
   DSA_REQUIRE(features * a.kdim * 4 < (int64_t(1) << 31), "the fp32 weights must be below 2 GiB");
   DSA_REQUIRE(reinterpret_cast<uintptr_t>(weight) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
               "the fp32 weights and their output must be 16-byte aligned");
-  NarrowArgs w = {};
-  w.hidden = a.hidden;
-  w.hidden_stride = a.hidden_stride;
-  w.weight = weight;
-  w.tokens = a.tokens;
-  w.features = (int32_t)features;
-  w.kdim = a.kdim;
-  w.parts = static_cast<float*>(parts);
-  if (int st = launch_narrow<true>(w, rope, s)) return st;
-  const int64_t quads = (int64_t)a.tokens * features / 4;
-  DSA_REQUIRE((quads + 255) / 256 <= 0x7fffffffLL, "problem too large");
-  hipLaunchKernelGGL(finish_weights_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, w.parts, w.splits,
-                     quads, scale, out);
-  return check_launch("finish_weights_kernel");
+  DSA_REQUIRE((int64_t)a.tokens * features * 4 < (int64_t(1) << 31), "the fp32 output must be below 2 GiB");
+  const int64_t slice = narrow_slice(a.tokens, a.kdim, features);
+  for (int64_t t0 = 0; t0 < a.tokens; t0 += slice) {
+    NarrowArgs w = {};
+    w.hidden = a.hidden + t0 * a.hidden_stride;
+    w.hidden_stride = a.hidden_stride;
+    w.weight = weight;
+    w.tokens = (int32_t)std::min<int64_t>(slice, a.tokens - t0);
+    w.features = (int32_t)features;
+    w.kdim = a.kdim;
+    w.parts = static_cast<float*>(parts);
+    if (int st = launch_narrow<true>(w, a.tokens, t0 == 0 ? rope : RopeTableArgs{}, s)) return st;
+    const int64_t quads = (int64_t)w.tokens * features / 4;
+    hipLaunchKernelGGL(finish_weights_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, w.parts, w.splits,
+                       quads, scale, out + t0 * features);
+    if (int st = check_launch("finish_weights_kernel")) return st;
+  }
+  return 0;
 }
 
 extern "C" int dsa_project_weights(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim,
@@ -1091,31 +1108,35 @@ int launch_encode_keys_gemm(const void* hidden, int64_t hidden_stride, int64_t t
   DSA_REQUIRE(((tokens - 1) * hidden_stride + kdim) * 2 < (int64_t(1) << 31) &&
                   kHeadDim * kdim * 2 < (int64_t(1) << 31),
               "hidden and wk must each be below 2 GiB");
-  NarrowArgs w = {};
-  w.hidden = static_cast<const uint16_t*>(hidden);
-  w.hidden_stride = hidden_stride;
-  w.weight = wk;
-  w.tokens = (int32_t)tokens;
-  w.features = kHeadDim;
-  w.kdim = (int32_t)kdim;
-  w.parts = static_cast<float*>(parts);
-  if (int st = launch_narrow<false>(w, RopeTableArgs{}, stream)) return st;
-  KeysArgs a = {};
-  a.parts = w.parts;
-  a.splits = w.splits;
-  a.tokens = (int32_t)tokens;
-  a.ln_weight = ln_weight;
-  a.ln_bias = ln_bias;
-  a.ln_bf16 = ln_bf16;
-  a.ln_eps = ln_eps;
-  a.positions = positions;
-  a.theta = theta;
-  a.out = static_cast<uint16_t*>(out);
-  a.out_stride = out_stride;
-  a.out_rows = out_rows;
-  a.out_row_limit = out_row_limit;
-  hipLaunchKernelGGL(finish_keys_kernel, dim3((unsigned)((tokens + 7) / 8)), dim3(256), 0, stream, a);
-  return check_launch("finish_keys_kernel");
+  const int64_t slice = narrow_slice(tokens, kdim, kHeadDim);
+  for (int64_t t0 = 0; t0 < tokens; t0 += slice) {
+    NarrowArgs w = {};
+    w.hidden = static_cast<const uint16_t*>(hidden) + t0 * hidden_stride;
+    w.hidden_stride = hidden_stride;
+    w.weight = wk;
+    w.tokens = (int32_t)std::min(slice, tokens - t0);
+    w.features = kHeadDim;
+    w.kdim = (int32_t)kdim;
+    w.parts = static_cast<float*>(parts);
+    if (int st = launch_narrow<false>(w, tokens, RopeTableArgs{}, stream)) return st;
+    KeysArgs a = {};
+    a.parts = w.parts;
+    a.splits = w.splits;
+    a.tokens = w.tokens;
+    a.ln_weight = ln_weight;
+    a.ln_bias = ln_bias;
+    a.ln_bf16 = ln_bf16;
+    a.ln_eps = ln_eps;
+    a.positions = positions + t0;
+    a.theta = theta;
+    a.out = static_cast<uint16_t*>(out) + (out_rows ? 0 : t0 * out_stride);
+    a.out_stride = out_stride;
+    a.out_rows = out_rows ? out_rows + t0 : nullptr;
+    a.out_row_limit = out_rows ? out_row_limit : w.tokens;
+    hipLaunchKernelGGL(finish_keys_kernel, dim3((unsigned)((w.tokens + 7) / 8)), dim3(256), 0, stream, a);
+    if (int st = check_launch("finish_keys_kernel")) return st;
+  }
+  return 0;
 }
 
 }  // namespace dsa

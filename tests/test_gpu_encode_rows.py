@@ -158,3 +158,55 @@ def test_wq_tiles_agree(device, kdim, strided) -> None:
     scale = hidden[-80:].double().abs() @ module.wq.weight.double().abs().t()
     # one rounding to bf16 (2^-9), fp32 sums of kdim products below 2^-20 of their magnitudes
     assert ((whole[-80:].double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * scale).all()
+
+
+def test_partial_sums_past_one_slice(device) -> None:
+    # 1100 tokens x 8192 fp32 features in three splits of k: 96 KiB of partial
+    # sums a token, so two slices; 131089 keys in one split: two slices as well.
+    gen = torch.Generator().manual_seed(41)
+    tokens, kdim, features = 1100, 264, 8192
+    print(f"project weights slices tokens={tokens} kdim={kdim} features={features}", flush=True)
+    hidden = torch.randn(tokens, kdim, generator=gen).to(device, torch.bfloat16)
+    weight = (torch.randn(features, kdim, generator=gen) * kdim**-0.5).to(device)
+    need = int(_lib.query("dsa_project_weights_workspace_bytes", tokens, kdim, features))
+    assert need <= 64 << 20
+    ws = torch.empty(need, device=device, dtype=torch.uint8)
+    out = torch.empty(tokens, features, device=device)
+    _lib.call("dsa_project_weights", hidden.data_ptr(), kdim, tokens, kdim, weight.data_ptr(), features, 0.5,
+              out.data_ptr(), ws.data_ptr(), need, _stream())
+    ref = 0.5 * (hidden.double() @ weight.double().t())
+    size = 0.5 * (hidden.double().abs() @ weight.double().abs().t())
+    assert ((out.double() - ref).abs() <= 2.0**-20 * size).all()
+
+    tokens = 131089
+    print(f"encode keys slices tokens={tokens}", flush=True)
+    module = sidecar.LightningIndexerSidecar(hidden_size=64, heads=2).to(device=device, dtype=torch.bfloat16).eval()
+    hidden = torch.randn(tokens, 64, generator=gen).to(device, torch.bfloat16)
+    positions = torch.arange(tokens, device=device)
+    whole = module.encode_keys(hidden, positions)
+    rows = torch.randperm(tokens, generator=gen).to(device)
+    cache = module.encode_keys(hidden, positions, out=torch.zeros_like(whole), out_rows=rows)
+    assert torch.equal(cache[rows].view(torch.int16), whole.view(torch.int16))
+    for a, b in ((0, 65536), (65536, tokens)):
+        part = module.encode_keys(hidden[a:b], positions[a:b])
+        assert torch.equal(whole[a:b].view(torch.int16), part.view(torch.int16)), a
+
+
+def test_fp32_module_keeps_partial_sums_small(device) -> None:
+    # wq of an fp32 module on bf16 hidden states, 2048 x 8192 outputs (64 MiB):
+    # beyond the projections, the rotated queries and the two weight arrays the
+    # call takes at most the 64 MiB of partial sums.
+    print("fp32 module peak memory", flush=True)
+    module = sidecar.LightningIndexerSidecar(hidden_size=2048).to(device).eval()
+    hidden = torch.randn(2048, 2048, generator=torch.Generator().manual_seed(5)).to(device, torch.bfloat16)
+    positions = torch.arange(2048, device=device)
+    module.encode_queries(hidden[:64], positions[:64])
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    queries, weights = module.encode_queries(hidden, positions)
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated() - before
+    own = 2 * (queries.numel() + weights.numel()) * 4
+    print(f"  peak {peak / 2**20:.0f} MiB, of it results and projections {own / 2**20:.0f} MiB", flush=True)
+    assert peak <= own + (64 << 20) + (1 << 20)
