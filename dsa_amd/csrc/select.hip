@@ -493,28 +493,38 @@ __device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, ui
 // ---------------------------------------------------------------------------
 // The usual case, with the entries in registers from the kernel's one round
 // trip of loads.  Every list holds all of its chunk's keys at or above
-// `origin`, the highest of the lists' lowest bins, so a k-th largest listed key
-// at or above it is the row's.  The entries are counted into bins of 2^11 keys
-// from there up, over an octave (above: the last bin): fine enough
-// that the cut's bin holds a few entries, so the entries of that bin, ranked
-// by every wave for itself, give the cut, where the 12-bit bins of the lists
-// leave 450 to 1,100 entries that took one or two more counting passes, and
-// whose counters serialised the first pass's atomics.  Five barriers in all.
+// `origin`, the highest of the lists' lowest bins (a list of the whole chunk
+// misses nothing), so a k-th largest listed key at or above it is the row's.
+// The entries are counted into bins of 2^12 keys over the octave above the
+// origin and of 2^21 keys from there up, and again inside the cut's bin, from
+// the registers, while that holds more than 64 entries (twice at most).  The
+// entries of the last bin, ranked by every wave for itself, give the cut; more
+// than 64 equal to it are taken in index order.
+// Scores are signed sums, so a cut near zero, where an octave of keys is a
+// sliver of scores, is as common as one in the octave above the origin; the
+// coarse bins hold those with at most one more count.  (Bins over that octave
+// alone sent k of L / 2, and one row in a few at k = 2048, to the general path
+// below, which costs 3 to 6 us more.  Bins that follow the row's range need its
+// largest key before the first count, 0.4 us of latency.)
 // Returns false, before anything is written, when a list is longer than the
-// registers hold, fewer than k keys lie at or above the origin (a list may
-// miss keys), or the cut lies past the octave or in a bin of more than 64
-// entries (ties).
+// registers hold or fewer than k keys lie at or above the origin (a list may
+// miss keys).  in_regs: how many of `pre` hold the list's entries then.
 //
 // Bound by latency: the loads' round trip, five barriers and a few hundred
-// VALU instructions a wave, one wave per SIMD.  Counting the 12-bit bins and a
-// radix cut from 8-byte entries -> this, MI355X: 1 x 4096 k 256 6.6 -> 5.4 us;
-// 5 x 20011 k 2048 9.7 -> 7.3; 16 x 32768 k 2048 9.6 -> 7.0; 4 x 131072 k 2048
-// (fp8) 11.4 -> 7.5.  From 8-byte entries with these bins: 6.0, 6.8, 6.8, 8.8.
+// VALU instructions a wave, one wave per SIMD; each further count adds a
+// microsecond.  Whole decode calls, MI355X, with 12-bit bins and a radix cut ->
+// with bins over one octave and the general path beyond -> this: 1 x 4096 k 256
+// 15.0 -> 13.4 -> 13.6 us; 5 x 20011 k 256 17.8 -> 16.5 -> 16.7; 16 x 32768 k
+// 2048 35.6 -> 37.4 -> 33.1; 5 x 20011 k 2048 18.9 -> 23.2 -> 18.9; 4 x 4096 k
+// 2048 17.4 -> 20.2 -> 16.0, of 100 equal keys each 19.5 -> 24.1 -> 16.8.
 // ---------------------------------------------------------------------------
-constexpr int kFineShift = 11;
+constexpr int kFineShift = 12;    // fine bins of 2^12 keys
+constexpr int kFineBins = 2048;   // over 2^23 keys: an octave
+constexpr int kCoarseShift = 21;  // then of 2^21
+constexpr int kCoarseBase = kFineBins - (kFineBins >> (kCoarseShift - kFineShift));
 
 __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared& sh, BufferRsrc words, uint32_t lbase,
-                                                  uint4 (&pre)[kListVecs], uint32_t list_len,
+                                                  uint4 (&pre)[kListVecs], int& in_regs, uint32_t list_len,
                                                   uint32_t list_bin, uint32_t own_pos, uint32_t j, uint32_t r,
                                                   uint32_t tpl, uint32_t row, uint32_t c) {
   const uint32_t tid = threadIdx.x;
@@ -522,10 +532,14 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
   const uint32_t wave = tid / kWave;
   const uint32_t kk = (uint32_t)a.k;
   const uint32_t ck = (uint32_t)a.chunk_keys;
+  auto clear_hist = [&] {
 #pragma unroll
-  for (int q = 0; q < kSelectBins / 4 / kSelThreads; ++q)
-    reinterpret_cast<uint4*>(sh.hist)[tid + kSelThreads * q] = make_uint4(0u, 0u, 0u, 0u);
+    for (int q = 0; q < kSelectBins / 4 / kSelThreads; ++q)
+      reinterpret_cast<uint4*>(sh.hist)[tid + kSelThreads * q] = make_uint4(0u, 0u, 0u, 0u);
+  };
+  clear_hist();
   if (tid == 0) sh.crowd = 0;
+  in_regs = a.loads;
   const uint32_t wbin = wave_max_u32(list_bin);  // (threads with no list read length and bin 0)
   const uint32_t wlen = wave_max_u32(list_len);
   if (lane == 0) {
@@ -541,7 +555,6 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
   }
   if (longest > 4u * tpl * kListVecs) return false;
   const int nq = __builtin_amdgcn_readfirstlane((int)((longest + 4u * tpl - 1u) / (4u * tpl)));
-  const uint32_t origin = top_bin << 20;
   uint32_t* own_keys = reinterpret_cast<uint32_t*>(sh.stage);
   // f(entry's place in its list, key) over this thread's loads; keys past the
   // list's end read 0, which is below every key selected here.
@@ -562,6 +575,7 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
     for (int q = 0; q < kListVecs; ++q)
       if (q >= a.loads && q < nq) pre[q] = load_scores(words, lbase, 4u * (r + tpl * q), list_len);
   }
+  in_regs = nq;
 #pragma unroll
   for (int q = 0; q < kListVecs; ++q) {
     if (q < nq) {
@@ -575,27 +589,95 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
     }
   }
   if (j == c && r == 0) sh.base[0] = list_len;
-  each([&](uint32_t, uint32_t key) {
-    const uint32_t b = min((key - origin) >> kFineShift, (uint32_t)kSelectBins - 1u);
-    if (key >= max(origin, 1u))
-      __hip_atomic_fetch_add(&sh.hist[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  });
-  __syncthreads();
-  if (wave == 0) {
-    const Locate t = wave_locate<kSelectBins / kWave>(sh.hist, kk, false);
-    if (lane == 0) {
-      sh.bin = t.digit;
-      sh.want = t.rem;
-      sh.miss = t.count;
+  // The cut is the want-th largest of the keys in [lowest, lowest + reach].  One
+  // copy of the counting code serves every count: a second one beside it cost
+  // each call 0.7 us of instruction fetch.
+  uint32_t lowest = max(top_bin << 20, 1u);
+  uint32_t reach = 0xffffffffu;
+  uint32_t want = kk, crowd;
+  int shift = kFineShift, coarse_shift = kCoarseShift;
+  uint32_t coarse_base = (uint32_t)kCoarseBase;
+#pragma unroll 1
+  for (;;) {
+    each([&](uint32_t, uint32_t key) {
+      const uint32_t d = key - lowest;
+      const uint32_t b = min(d >> shift, (d >> coarse_shift) + coarse_base);
+      if (key >= lowest && d <= reach)
+        __hip_atomic_fetch_add(&sh.hist[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    });
+    __syncthreads();
+    if (wave == 0) {
+      const Locate t = wave_locate<kSelectBins / kWave>(sh.hist, want, false);
+      if (lane == 0) {
+        sh.bin = t.digit;
+        sh.want = t.rem;
+        sh.miss = t.count;
+      }
     }
+    __syncthreads();
+    const uint32_t bin = sh.bin;
+    crowd = sh.miss;
+    want = sh.want;
+    if (bin == kNoBin) return false;
+    const bool coarse = bin >= coarse_base + (uint32_t)(kFineBins - kCoarseBase);
+    const int width = coarse ? coarse_shift : shift;
+    lowest += (coarse ? bin - coarse_base : bin) << width;
+    reach = (1u << width) - 1u;
+    if (crowd <= (uint32_t)kWave || width == 0) break;
+    // Again inside the bin, with no coarse bins.
+    shift = max(0, width - 12);
+    coarse_shift = 31;
+    coarse_base = (uint32_t)kSelectBins;
+    clear_hist();
+    __syncthreads();
   }
-  __syncthreads();
-  const uint32_t bin = sh.bin;
-  const uint32_t crowd = sh.miss;
-  if (bin >= (uint32_t)kSelectBins - 1u || crowd > (uint32_t)kWave) return false;  // (kNoBin is past every bin)
-  const uint32_t lowest = origin + (bin << kFineShift);
+  const uint32_t own_n = sh.base[0];
+  const uint32_t per = (own_n + kSelThreads - 1) / kSelThreads;
+  const uint32_t first = min(own_n, tid * per);
+  const uint32_t last = min(own_n, first + per);
+  int64_t* oidx = a.out_idx + (size_t)row * kk;
+  float* oval = a.out_val ? a.out_val + (size_t)row * kk : nullptr;
+  const uint32_t* own_list = reinterpret_cast<const uint32_t*>(a.lists + (size_t)row * (uint32_t)a.length + c * ck);
+  const uint32_t own_room = min(ck, (uint32_t)a.length - c * ck);
+  auto write = [&](uint32_t slot, uint32_t i, uint32_t key) {
+    if (slot < kk) {  // always true for consistent counts; keeps writes in the row
+      oidx[slot] = (int64_t)(per == 1u ? own_pos : own_list[own_room + i]);
+      if (oval) oval[slot] = ordered_to_float(key);
+    }
+  };
+  // Chosen entries of the lists before this one, and of this list in index
+  // order, a contiguous run per thread; the counts are packed in pairs, each
+  // below 2^16 (the entries fit the registers).
+  if (crowd > (uint32_t)kWave) {
+    // Ties: every key above `lowest` and the first `want` equal to it.
+    uint32_t above = 0, ties = 0;
+    if (j < c) {
+      each([&](uint32_t, uint32_t key) {
+        above += key > lowest ? 0x10000u : 0u;
+        ties += key == lowest ? 0x10000u : 0u;
+      });
+    }
+    for (uint32_t i = first; i < last; ++i) {
+      above += own_keys[i] > lowest ? 1u : 0u;
+      ties += own_keys[i] == lowest ? 1u : 0u;
+    }
+    uint32_t above_total, ties_total;
+    const uint32_t above_at = block_excl_scan<kSelWaves>(above, sh.wsum[0], above_total);
+    const uint32_t ties_at = block_excl_scan<kSelWaves>(ties, sh.wsum[1], ties_total);
+    const uint32_t ties_before = min(want, ties_total >> 16);
+    const uint32_t own_ties = want - ties_before;
+    uint32_t tie = ties_at & 0xffffu;
+    uint32_t slot = (above_total >> 16) + ties_before + (above_at & 0xffffu) + min(tie, own_ties);
+    for (uint32_t i = first; i < last; ++i) {
+      const uint32_t key = own_keys[i];
+      if (key < lowest) continue;
+      if (key == lowest && tie++ >= own_ties) continue;
+      write(slot++, i, key);
+    }
+    return true;
+  }
   each([&](uint32_t s, uint32_t key) {
-    if (key - lowest < 1u << kFineShift && key != 0u)
+    if (key >= lowest && key - lowest <= reach)
       sh.cands[__hip_atomic_fetch_add(&sh.crowd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)] =
           select_composite(key, j * ck + s);
   });
@@ -603,44 +685,24 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
   const uint64_t x = sh.cands[min(lane, crowd - 1u)];
   uint32_t larger = 0;
   for (uint32_t i = 0; i < crowd; ++i) larger += sh.cands[i] > x ? 1u : 0u;
-  const uint64_t hit = __ballot(lane < crowd && larger + 1u == sh.want);
+  const uint64_t hit = __ballot(lane < crowd && larger + 1u == want);
   const int owner = (int)__builtin_ctzll(hit);  // composites are distinct: one lane
   const uint32_t cut = (uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), owner);
   const uint32_t cut_place = ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, owner);
   auto chosen = [&](uint32_t key, uint32_t place) { return key > cut || (key == cut && place <= cut_place); };
-  // Chosen entries of the lists before this one, and of this list in index
-  // order, a contiguous run per thread.
   uint32_t before = 0;
   if (j < c)
     each([&](uint32_t s, uint32_t key) { before += chosen(key, j * ck + s) ? 1u : 0u; });
-  const uint32_t own_n = sh.base[0];
-  const uint32_t per = (own_n + kSelThreads - 1) / kSelThreads;
-  const uint32_t first = min(own_n, tid * per);
-  const uint32_t last = min(own_n, first + per);
   uint32_t mine = 0;
   for (uint32_t i = first; i < last; ++i) mine += chosen(own_keys[i], c * ck + i) ? 1u : 0u;
-  uint32_t packed_total;  // both counts below 2^16: the entries fit the registers
+  uint32_t packed_total;
   const uint32_t packed = block_excl_scan<kSelWaves>((before << 16) | mine, sh.wsum[0], packed_total);
   uint32_t slot = (packed_total >> 16) + (packed & 0xffffu);
-  int64_t* oidx = a.out_idx + (size_t)row * kk;
-  float* oval = a.out_val ? a.out_val + (size_t)row * kk : nullptr;
-  const uint32_t* own_list = reinterpret_cast<const uint32_t*>(a.lists + (size_t)row * (uint32_t)a.length + c * ck);
-  const uint32_t own_room = min(ck, (uint32_t)a.length - c * ck);
   for (uint32_t i = first; i < last && mine; ++i) {
     const uint32_t key = own_keys[i];
     if (chosen(key, c * ck + i)) {
-      if (slot < kk) {  // always true for consistent counts; keeps writes in the row
-        oidx[slot] = (int64_t)(per == 1u ? own_pos : own_list[own_room + i]);
-        if (oval) oval[slot] = ordered_to_float(key);
-      }
-      ++slot;
+      write(slot++, i, key);
       --mine;
-    }
-  }
-  if (c == 0) {
-    for (uint32_t i = min((uint32_t)a.length, kk) + tid; i < kk; i += kSelThreads) {
-      oidx[i] = -1;
-      if (oval) oval[i] = -__builtin_inff();
     }
   }
   return true;
@@ -685,6 +747,23 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   const float* srow = a.scores + (size_t)row * n;
   const uint64_t* lrow = a.lists + (size_t)row * n;
   DSA_TRACE_MARK(g_trace_select, blockIdx.x, 0);
+  if (n <= kk) {
+    // Every key is chosen: the row's positions, then padding.
+    int64_t* oidx = a.out_idx + (size_t)row * kk;
+    float* oval = a.out_val ? a.out_val + (size_t)row * kk : nullptr;
+    for (uint32_t i = c * ck + tid; i < min(n, (c + 1u) * ck); i += kSelThreads) {
+      oidx[i] = (int64_t)i;
+      if (oval) oval[i] = ordered_to_float(float_to_ordered(srow[i]));
+    }
+    if (c == 0) {
+      for (uint32_t i = n + tid; i < kk; i += kSelThreads) {
+        oidx[i] = -1;
+        if (oval) oval[i] = -__builtin_inff();
+      }
+      if (a.count_parts && wave == 0) sum_count_parts(a, row, chunks);
+    }
+    return;
+  }
   // This thread's list j and its place r among the list's threads.
   const uint32_t tpl = chunks >= (uint32_t)kSelThreads ? 1u : (uint32_t)kSelThreads / chunks;
   const uint32_t j = tid / tpl;
@@ -704,24 +783,40 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   for (int q = 0; q < kListVecs; ++q)
     pre[q] = load_scores(words, lbase, 4u * (r + tpl * q), q < a.loads ? chunk_len : 0u);
   const uint32_t list_len = min(m.x, chunk_len);  // (keeps every read inside the row whatever the workspace holds)
-  const uint32_t list_bin = m.y;
-  if (select_lists_fast(a, sh, words, lbase, pre, list_len, list_bin, own_pos, j, r, tpl, row, c)) {
+  // A list of the whole chunk misses nothing, wherever it stops.
+  const uint32_t list_bin = list_len < chunk_len ? m.y : 0u;
+  int in_regs;  // entries 4 (r + tpl q) .. + 3, q < in_regs, are in pre
+  if (select_lists_fast(a, sh, words, lbase, pre, in_regs, list_len, list_bin, own_pos, j, r, tpl, row, c)) {
     if (a.count_parts && c == 0 && wave == 0) sum_count_parts(a, row, chunks);
     DSA_TRACE_MARK(g_trace_select, blockIdx.x, 4);
     return;
   }
   if (a.count_parts && c == 0 && wave == 0) sum_count_parts(a, row, chunks);
   __syncthreads();  // the shared arrays are taken over below
-  bool raw = false;
-  auto load_entry = [&](uint32_t s) -> uint64_t {  // entry s of this thread's source
-    const uint32_t pos = j * ck + s;
-    return select_composite(raw ? float_to_ordered(srow[pos]) : lwords[s], pos);
-  };
+  // A row that fits the stage is read raw at once: that costs less than finding
+  // out which lists miss keys.
+  bool raw = n <= (uint32_t)kListStageCapacity;
 
   uint32_t entries = 0;
   uint32_t src_len = 0;
   uint32_t src_base = 0;
   bool staged = false;
+  // f(s, entry) over this thread's share of its source's entries from `from`
+  // on, eight loads in flight.
+  auto each_entry = [&](uint32_t from, auto&& f) {
+    const uint32_t* source = raw ? reinterpret_cast<const uint32_t*>(srow + j * ck) : lwords;
+#pragma unroll 1
+    for (uint32_t s0 = from + r; s0 < src_len; s0 += 8u * tpl) {
+      uint32_t v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = source[min(s0 + tpl * i, src_len - 1u)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t s = s0 + tpl * i;
+        if (s < src_len) f(s, select_composite(raw ? float_to_ordered(__uint_as_float(v[i])) : v[i], j * ck + s));
+      }
+    }
+  };
 #pragma unroll 1
   for (int round = 0; round < 2; ++round) {
 #pragma unroll
@@ -745,7 +840,18 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
       __hip_atomic_fetch_add(&sh.hist[(uint32_t)(x >> 52)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (staged) sh.stage[src_base + s] = x;
     };
-    for (uint32_t s = r; s < src_len; s += tpl) take(s, load_entry(s));
+    if (!raw) {
+#pragma unroll
+      for (int q = 0; q < kListVecs; ++q) {
+        if (q >= in_regs) continue;
+        const uint32_t s = 4u * (r + tpl * q);
+        const uint32_t keys[4] = {pre[q].x, pre[q].y, pre[q].z, pre[q].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (s + i < src_len) take(s + i, select_composite(keys[i], j * ck + s + i));
+      }
+    }
+    each_entry(raw ? 0u : 4u * tpl * in_regs, take);
     __syncthreads();
     if (wave == 0) {
       const Locate t = wave_locate<kSelectBins / kWave>(sh.hist, kk, true);
@@ -770,11 +876,12 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
   const uint32_t bin = sh.bin;
   auto raw_of = [&](uint32_t list) { return sh.raw[list] != 0u; };
   // Entries of the sources before this chunk's: those above the cut's bin
-  // are chosen; those inside it are compacted with the rest of the bin.
-  // (With at most k entries, every entry of the earlier sources is chosen.)
-  uint32_t before = (bin == kNoBin && tid == 0) ? sh.base[c] : 0u;
-  uint64_t cstar = uint64_t(1) << 32;  // every listed key when they number at most k
-  if (bin != kNoBin && staged) {
+  // are chosen; those inside it are compacted with the rest of the bin.  (The
+  // row has more than k keys, and at most k entries miss some of them: there
+  // is a bin.)
+  uint32_t before = 0;
+  uint64_t cstar;
+  if (staged) {
     // Staged entries: the radix cut runs over the whole stage, counting only
     // the cut bin's entries (its prefix), with no compaction of the bin
     // first (a count, a scan and a placement, 0.6 us at C2); then the chosen
@@ -784,27 +891,25 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
     __syncthreads();
     cstar = radix_cut<true>(bin, sh.want, entries, [&](uint32_t i) { return sh.stage[i]; }, digits, sh.radix);
     DSA_TRACE_MARK(g_trace_select, blockIdx.x, 2);
-    before = 0;
     for (uint32_t i = tid; i < sh.base[c]; i += kSelThreads) before += sh.stage[i] >= cstar ? 1u : 0u;
-  } else if (bin != kNoBin) {
+  } else {
     // Entries read in place (more than the stage holds): count, scan, then
     // place the entries of the cut's bin.
     uint32_t n_cand = 0;
-    for (uint32_t s = r; s < src_len; s += tpl) {
-      const uint32_t b = (uint32_t)(load_entry(s) >> 52);
+    each_entry(0u, [&](uint32_t, uint64_t x) {
+      const uint32_t b = (uint32_t)(x >> 52);
       n_cand += b == bin ? 1u : 0u;
       before += (b > bin && j < c) ? 1u : 0u;
-    }
+    });
     uint32_t crowd_total;
     uint32_t slot = block_excl_scan<kSelWaves>(n_cand, sh.wsum[0], crowd_total);
     if (n_cand) {
-      for (uint32_t s = r; s < src_len; s += tpl) {
-        const uint64_t x = load_entry(s);
+      each_entry(0u, [&](uint32_t, uint64_t x) {
         if ((uint32_t)(x >> 52) == bin) {
           if (slot < (uint32_t)kCandCapacity) sh.cands[slot] = x;
           ++slot;
         }
-      }
+      });
     }
     if (tid == 0) sh.crowd = crowd_total;
     // The bin counters are dead: they become the radix digit counters.
@@ -877,12 +982,6 @@ __global__ __launch_bounds__(kSelThreads) void select_lists_kernel(ListArgs a) {
       }
       ++slot;
       --mine;
-    }
-  }
-  if (c == 0) {
-    for (uint32_t i = min(n, kk) + tid; i < kk; i += kSelThreads) {
-      oidx[i] = -1;
-      if (oval) oval[i] = -__builtin_inff();
     }
   }
   DSA_TRACE_MARK(g_trace_select, blockIdx.x, 4);
