@@ -443,21 +443,30 @@ __global__ __launch_bounds__(THREADS) void topk_kernel(TopkArgs a) {
 //  - Bins are linear in the order key between the row's least finite and its
 //    largest key: an eighth of an octave wide for scores around zero, finer
 //    for scores that share an offset, and monotone, so the bound (a bin's
-//    lower edge) never splits equal keys.
+//    lower edge) never splits equal keys.  -inf is not counted: its lanes all
+//    met in one counter (1 x 32768, 95 % -inf, k 256: 18.1 -> 11.8 us).
 //  - The sample's rank is k / 4 + 4 sqrt(k / 4) + 4, four and a half standard
-//    deviations above the quarter of the top k it holds on average: when it
-//    still leaves fewer than k candidates, or a crowded bin leaves more than
-//    fit, the row takes the radix select over all elements.
+//    deviations above the quarter of the top k it holds on average.
 //  - Up to 128 candidates are ranked against each other.  More are binned
 //    again, linearly in the key from the bound up, which leaves a few in a
 //    bin: in index order, the cut's bin is resolved by ranking its members; a
 //    sorted result is a counting sort by bin whose members order themselves.
-//    A bin of more than 64 leaves the row to the radix select.
+//  - Where more than 64 share the cut's bin, the bin alone is counted again, 12
+//    bits at a time, down to one key, whose ties are taken in index order.  The
+//    same from the row, read again, where the bound leaves too many or too few
+//    (a sample that missed the top, a cut at -inf).  A radix select over every
+//    key of the row, as before, sent all of them through shared counters: 1 x
+//    4096 of one value, k 256, 31.9 -> 13.7 us, 1 x 32768 of some twenty values,
+//    27.6 -> 15.5.
+//  - Rows of at most k elements are written, or sorted, as they are: 1 x 1000,
+//    k 1000, 6.7 -> 3.4 us.
 //
-// 512 rows of 32768, k = 2048, index order: 68 us -> 32.5 us (two rounds of
+// 512 rows of 32768, k = 2048, index order: 68 us -> 32 us (two rounds of
 // one workgroup per CU: 128 registers past 16384 elements); 100 rows of 16384:
 // 16.9 -> 11.0; one row of 32768, k = 2048, sorted: 42.5 -> 14.9 us, of 4096:
-// 26.5 -> 10.1 us (the bitonic sort took 66 barriers).
+// 26.8 -> 9.6 us (the bitonic sort took 66 barriers).  Of 288 shapes (rows of
+// random, bf16, tied, constant and partly -inf scores) none is slower than with
+// topk_kernel or the distributed select.
 // ---------------------------------------------------------------------------
 constexpr int kRowBins = 4096;
 constexpr int kRowPairs = 128;       // candidates ranked pairwise
@@ -479,6 +488,14 @@ struct RowShared {
 
 // Shift that brings keys up to `span` above their origin into kRowBins bins.
 __device__ __forceinline__ int bin_shift(uint32_t span) { return max(0, 20 - (int)__clz((int)(span | 1u))); }
+
+// Padding of a row's output from place `from` on.
+__device__ __forceinline__ void pad_row(const TopkArgs& a, int64_t out_base, int from, int tid) {
+  for (int i = from + tid; i < a.k; i += kTopkThreads) {
+    if (a.out_idx) a.out_idx[out_base + i] = -1;
+    if (a.out_val) a.out_val[out_base + i] = -__builtin_inff();
+  }
+}
 
 template <int EPT, int CAP>
 __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) void topk_rows_kernel(TopkArgs a) {
@@ -506,9 +523,8 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
   // has key 0 as well, the NaN 0xffffffff: such an element is no candidate, as
   // in topk_kernel, so a row may hold fewer than k keys also where n > k, and
   // the output is padded from the number of keys found.
-  uint32_t key[EPT];
   auto pos_of = [&](int e) { return kStep * (e >> 2) + 4 * tid + (e & 3); };
-  {
+  auto load = [&](const float* scores, int n, uint32_t (&key)[EPT]) {
     const BufferRsrc rsrc = make_buffer(scores, (uint32_t)n * 4u);
 #pragma unroll
     for (int c = 0; c < EPT / 4; ++c) {
@@ -519,200 +535,292 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
       key[4 * c + 2] = raw.z;
       key[4 * c + 3] = raw.w;
     }
-  }
-  reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
-  sh.bits[tid] = 0;
-  if (tid < kRowPairs) sh.rank[tid] = 0;
-  if (tid == 0) sh.near_n = 0;
+  };
+  auto order = [&](int n, uint32_t (&key)[EPT]) {
 #pragma unroll
-  for (int e = 0; e < EPT; ++e)
-    key[e] = pos_of(e) < n ? float_to_ordered(__uint_as_float(key[e])) : 0u;
+    for (int e = 0; e < EPT; ++e)
+      key[e] = pos_of(e) < n ? float_to_ordered(__uint_as_float(key[e])) : 0u;
+  };
 
-  bool done = false;  // sorted output written
-  if (n <= k) {
-    // Every element with a key is chosen.
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < EPT; e += 4) {
-      uint32_t set = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) set |= key[e + i] != 0 ? 1u << i : 0u;
-      if (set) atomicOr(&sh.bits[pos_of(e) >> 5], set << (pos_of(e) & 31));
-    }
-  } else {
-    uint32_t lo = 0xffffffffu, hi = 0u;
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      lo = min(lo, key[e] > kNegInfKey ? key[e] : 0xffffffffu);
-      hi = max(hi, key[e]);
-    }
-    lo = wave_min_u32(lo);
-    hi = wave_max_u32(hi);
-    if (lane == 0) {
-      sh.wave_lo[wave] = lo;
-      sh.wave_hi[wave] = hi;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      lo = min(lo, sh.wave_lo[i]);
-      hi = max(hi, sh.wave_hi[i]);
-    }
-    lo = min(lo, hi);
-    const int shift = bin_shift(hi - lo);
-#pragma unroll
-    for (int e = 0; e < EPT; e += kSample ? 4 : 1) {
-      if (kStep * (e >> 2) >= n) break;
-      if (pos_of(e) < n) lds_add(&sh.bins[key[e] <= lo ? 0u : (key[e] - lo) >> shift], 1u);
-    }
-    __syncthreads();
-    if (wave == 0) {
-      uint32_t want = (uint32_t)k;
-      if (kSample) {
-        const float quarter = 0.25f * (float)k;
-        want = min((uint32_t)(quarter + 4.f * sqrtf(quarter)) + 4u, (uint32_t)((n + 3) / 4));
-      }
-      const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, want, false);
-      if (lane == 0) sh.digit = loc.digit;
-    }
-    __syncthreads();
-    const uint32_t digit = sh.digit;
-    const uint32_t bound = digit == 0 ? 1u : lo + (digit << shift);
-    // Candidates: every key at or above the bound.
-    uint32_t mine = 0;
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) mine += (uint32_t)__popcll(__ballot(key[e] >= bound));
-    if (lane == 0) sh.ws[0][wave] = mine;
+  bool done = false;      // sorted output written
+  bool resolved = false;  // sh.bits holds the chosen positions
+  int to_sort = 0;        // or else sh.cand the candidates of a sorted output, if any
+  uint32_t lo = 1u, hi = 1u, bound = 1u, lowest, reach, want, m;
+  auto candidates = [&] { return m <= (uint32_t)CAP && m >= (uint32_t)k; };
+  {
+    uint32_t key[EPT];
+    load(scores, n, key);
     reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
-    __syncthreads();
-    uint32_t at = 0, m = 0;
+    sh.bits[tid] = 0;
+    if (tid < kRowPairs) sh.rank[tid] = 0;
+    if (tid == 0) sh.near_n = 0;
+    order(n, key);
+    if (EPT == 4 && n <= k) {
+      // Every element with a key is chosen: in most rows, every element.  (A
+      // short last chunk of a long row takes the general way.)
+      bool keyless = false;
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      const uint32_t c = sh.ws[0][i];
-      at += i < wave ? c : 0u;
-      m += c;
+      for (int e = 0; e < 4; ++e) keyless |= key[e] == 0 && pos_of(e) < n;
+      if (!__syncthreads_or(keyless)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int p = pos_of(e);
+          if (p >= n) continue;
+          if (a.sorted) {
+            sh.cand[p] = composite(key[e], p);
+            continue;
+          }
+          if (a.out_idx) a.out_idx[out_base + p] = start + (int64_t)p;
+          if (a.out_val) a.out_val[out_base + p] = scores[p];
+        }
+        m = (uint32_t)n;
+        to_sort = n;
+      }
     }
-    at = __builtin_amdgcn_readfirstlane(at);
-    bool resolved = false;
-    if (m >= (uint32_t)k && m <= (uint32_t)CAP) {
+    if (to_sort == 0) {
+      // [lo, hi]: from the least finite key (the largest key of a row without one)
+      // to the largest.
+      lo = 0xffffffffu;
+      hi = 1u;
 #pragma unroll
       for (int e = 0; e < EPT; ++e) {
-        const bool in = key[e] >= bound;
-        const uint64_t mask = __ballot(in);
-        if (in) sh.cand[at + lanes_below(mask)] = composite(key[e], pos_of(e));
-        at += (uint32_t)__popcll(mask);
+        lo = min(lo, key[e] > kNegInfKey ? key[e] : 0xffffffffu);
+        hi = max(hi, key[e]);
+      }
+      lo = wave_min_u32(lo);
+      hi = wave_max_u32(hi);
+      if (lane == 0) {
+        sh.wave_lo[wave] = lo;
+        sh.wave_hi[wave] = hi;
       }
       __syncthreads();
-      if (m <= (uint32_t)kRowPairs) {
-        // Rank by pairwise comparison: `width` candidates, the threads past
-        // them each a further part of the comparisons.
-        int width = kWave;
-        while (width < (int)m) width <<= 1;
-        const int parts = kTopkThreads / width;
-        const int ci = tid & (width - 1);
-        const int per = ((int)m + parts - 1) / parts;
-        const int j0 = tid / width * per;
-        const int j1 = min((int)m, j0 + per);
-        const uint64_t c = sh.cand[min(ci, (int)m - 1)];
-        uint32_t larger = 0;
-#pragma unroll 8
-        for (int j = j0; j < j1; ++j) larger += sh.cand[j] > c ? 1u : 0u;
-        if (ci < (int)m) lds_add(&sh.rank[ci], larger);
-        __syncthreads();
-        if (tid < (int)m && sh.rank[tid] < (uint32_t)k) {
-          const uint64_t mine64 = sh.cand[tid];
-          const uint32_t p = ~(uint32_t)mine64;
-          if (a.sorted) {
-            const int64_t slot = out_base + sh.rank[tid];
-            if (a.out_idx) a.out_idx[slot] = start + (int64_t)p;
-            if (a.out_val) a.out_val[slot] = scores[p];
-          } else {
-            atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
-          }
-        }
-        done = a.sorted != 0;
-        resolved = true;
-      } else {
-        // Bins from the bound up, over the candidates alone.
-        const int shift2 = bin_shift(hi - bound);
-        uint64_t c[CAP / kTopkThreads];
 #pragma unroll
-        for (int i = 0; i < CAP / kTopkThreads; ++i) {
-          const int j = tid + kTopkThreads * i;
-          c[i] = j < (int)m ? sh.cand[j] : 0u;
-          if (c[i]) lds_add(&sh.bins[((uint32_t)(c[i] >> 32) - bound) >> shift2], 1u);
+      for (int i = 0; i < kWaves; ++i) {
+        lo = min(lo, sh.wave_lo[i]);
+        hi = max(hi, sh.wave_hi[i]);
+      }
+      lo = min(lo, hi);
+      // Candidates: the m keys at or above `bound`.
+      bound = n > k ? lo : 1u;  // (n <= k: some elements have no key)
+      if (n > k && lo < hi) {
+        const int shift = bin_shift(hi - lo);
+#pragma unroll
+        for (int e = 0; e < EPT; e += kSample ? 4 : 1) {
+          if (kStep * (e >> 2) >= n) break;
+          if (key[e] >= lo) lds_add(&sh.bins[(key[e] - lo) >> shift], 1u);
         }
         __syncthreads();
+        if (wave == 0) {
+          uint32_t rank = (uint32_t)k;
+          if (kSample) {
+            const float quarter = 0.25f * (float)k;
+            rank = (uint32_t)(quarter + 4.f * sqrtf(quarter)) + 4u;
+          }
+          const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, rank, false);
+          if (lane == 0) sh.digit = loc.digit == kNoBin ? 0u : loc.digit;  // (fewer finite keys: all of them)
+        }
+        __syncthreads();
+        bound += sh.digit << shift;
+        reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+      }
+      uint32_t mine = 0;
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) mine += (uint32_t)__popcll(__ballot(key[e] >= bound));
+      if (lane == 0) sh.ws[0][wave] = mine;
+      __syncthreads();
+      uint32_t at = 0;
+      m = 0;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        const uint32_t c = sh.ws[0][i];
+        at += i < wave ? c : 0u;
+        m += c;
+      }
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (candidates()) {
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) {
+          const bool in = key[e] >= bound;
+          const uint64_t mask = __ballot(in);
+          if (in) sh.cand[at + lanes_below(mask)] = composite(key[e], pos_of(e));
+          at += (uint32_t)__popcll(mask);
+        }
+      }
+    }
+  }
+  // The cut is the want-th largest of the keys in [lowest, lowest + reach].
+  lowest = bound;
+  reach = hi - bound;
+  want = (uint32_t)k;
+  // Counts the keys in [lowest, lowest + reach] again, 12 bits a time, down to
+  // the cut's key, and sets the bits of the keys above it and of its first ties
+  // in index order; `each` passes every (key, position) of this thread.
+  auto narrow = [&](auto&& each) {
+    const uint32_t end = lowest + reach;
+#pragma unroll 1
+    while (reach) {
+      const int shift = bin_shift(reach);
+      __syncthreads();
+      reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+      __syncthreads();
+      each([&](uint32_t x, int) {
+        if (x >= lowest && x - lowest <= reach) lds_add(&sh.bins[(x - lowest) >> shift], 1u);
+      });
+      __syncthreads();
+      if (wave == 0) {
+        const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, want, false);
+        if (lane == 0) {
+          sh.digit = loc.digit;
+          sh.rem = loc.rem;
+        }
+      }
+      __syncthreads();
+      lowest += sh.digit << shift;
+      want = sh.rem;
+      reach = min((1u << shift) - 1u, end - lowest);
+    }
+    __syncthreads();
+    uint32_t* ties = sh.bins;  // one word per thread
+    ties[tid] = 0;
+    __syncthreads();
+    each([&](uint32_t x, int p) {
+      if (x >= lowest) atomicOr(x > lowest ? &sh.bits[p >> 5] : &ties[p >> 5], 1u << (p & 31));
+    });
+    __syncthreads();
+    uint32_t word = ties[tid];
+    uint32_t total;
+    const uint32_t before = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[0], total);
+    int take = (int)want - (int)before;  // this word's ties that are chosen, lowest first
+    uint32_t chosen = 0;
+    while (word && take > 0) {
+      chosen |= word & (0u - word);
+      word &= word - 1;
+      --take;
+    }
+    sh.bits[tid] |= chosen;
+  };
+  if (to_sort == 0 && candidates()) {
+    __syncthreads();
+    if (m <= (uint32_t)kRowPairs) {
+      // Rank by pairwise comparison: `width` candidates, the threads past
+      // them each a further part of the comparisons.
+      int width = kWave;
+      while (width < (int)m) width <<= 1;
+      const int parts = kTopkThreads / width;
+      const int ci = tid & (width - 1);
+      const int per = ((int)m + parts - 1) / parts;
+      const int j0 = tid / width * per;
+      const int j1 = min((int)m, j0 + per);
+      const uint64_t c = sh.cand[min(ci, (int)m - 1)];
+      uint32_t larger = 0;
+#pragma unroll 8
+      for (int j = j0; j < j1; ++j) larger += sh.cand[j] > c ? 1u : 0u;
+      if (ci < (int)m) lds_add(&sh.rank[ci], larger);
+      __syncthreads();
+      if (tid < (int)m && sh.rank[tid] < (uint32_t)k) {
+        const uint32_t p = ~(uint32_t)sh.cand[tid];
         if (a.sorted) {
-          // Counting sort by bin, largest first; a bin's few members order
-          // themselves.  A crowded bin leaves the row to the radix select.
-          uint32_t b[4], sum = 0, most = 0;
+          const int64_t slot = out_base + sh.rank[tid];
+          if (a.out_idx) a.out_idx[slot] = start + (int64_t)p;
+          if (a.out_val) a.out_val[slot] = scores[p];
+        } else {
+          atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
+        }
+      }
+      done = a.sorted != 0;
+      resolved = true;
+    } else {
+      // Bins from the bound up, over the candidates alone.
+      const int shift = bin_shift(hi - bound);
+      auto bin_of = [&](uint64_t c) { return ((uint32_t)(c >> 32) - bound) >> shift; };
+      bool crowded = false;
+      uint64_t c[CAP / kTopkThreads];
+#pragma unroll
+      for (int i = 0; i < CAP / kTopkThreads; ++i) {
+        const int j = tid + kTopkThreads * i;
+        c[i] = j < (int)m ? sh.cand[j] : 0u;
+        if (c[i]) lds_add(&sh.bins[bin_of(c[i])], 1u);
+      }
+      auto each_candidate = [&](auto&& f) {
+#pragma unroll
+        for (int i = 0; i < CAP / kTopkThreads; ++i) f((uint32_t)(c[i] >> 32), (int)~(uint32_t)c[i]);
+      };
+      __syncthreads();
+      if (a.sorted) {
+        // Counting sort by bin, largest first; a bin's few members order
+        // themselves.  With a crowded bin the candidates, or the top k of many
+        // more, are sorted by comparison.
+        uint32_t b[4], sum = 0, most = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          b[i] = sh.bins[kRowBins - 1 - 4 * tid - i];
+          sum += b[i];
+          most = max(most, b[i]);
+        }
+        if (most > (uint32_t)kWave) sh.near_n = 1;
+        uint32_t total;
+        uint32_t at2 = block_excl_scan<kWaves>(sum, sh.ws[1], total);
+        if (sh.near_n == 0) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            b[i] = sh.bins[kRowBins - 1 - 4 * tid - i];
-            sum += b[i];
-            most = max(most, b[i]);
-          }
-          if (most > (uint32_t)kWave) sh.near_n = 1;
-          uint32_t total;
-          uint32_t at2 = block_excl_scan<kWaves>(sum, sh.ws[1], total);
-          if (sh.near_n == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              sh.bins[kRowBins - 1 - 4 * tid - i] = at2;
-              at2 += b[i];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < CAP / kTopkThreads; ++i)
-              if (c[i]) sh.cand[atomicAdd(&sh.bins[((uint32_t)(c[i] >> 32) - bound) >> shift2], 1u)] = c[i];
-            __syncthreads();
-#pragma unroll 1
-            for (int j = tid; j < (int)m; j += kTopkThreads) {
-              const uint64_t x = sh.cand[j];
-              const uint32_t bin = ((uint32_t)(x >> 32) - bound) >> shift2;
-              int slot = j;
-              for (int q = j - 1; q >= 0; --q) {
-                const uint64_t y = sh.cand[q];
-                if (((uint32_t)(y >> 32) - bound) >> shift2 != bin) break;
-                slot -= y < x ? 1 : 0;
-              }
-              for (int q = j + 1; q < (int)m; ++q) {
-                const uint64_t y = sh.cand[q];
-                if (((uint32_t)(y >> 32) - bound) >> shift2 != bin) break;
-                slot += y > x ? 1 : 0;
-              }
-              if (slot < k) {
-                const uint32_t p = ~(uint32_t)x;
-                if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)p;
-                if (a.out_val) a.out_val[out_base + slot] = scores[p];
-              }
-            }
-            done = true;
-            resolved = true;
-          }
-        } else {
-          if (wave == 0) {
-            const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, (uint32_t)k, false);
-            if (lane == 0) {
-              sh.digit = loc.digit;
-              sh.rem = loc.rem;
-              sh.count = loc.count;
-            }
+            sh.bins[kRowBins - 1 - 4 * tid - i] = at2;
+            at2 += b[i];
           }
           __syncthreads();
-        }
-        if (!a.sorted && sh.count <= (uint32_t)kWave) {
-          const uint32_t cut = sh.digit;
 #pragma unroll
           for (int i = 0; i < CAP / kTopkThreads; ++i)
-            if (c[i] && ((uint32_t)(c[i] >> 32) - bound) >> shift2 == cut) sh.near[atomicAdd(&sh.near_n, 1u)] = c[i];
+            if (c[i]) sh.cand[atomicAdd(&sh.bins[bin_of(c[i])], 1u)] = c[i];
+          __syncthreads();
+#pragma unroll 1
+          for (int j = tid; j < (int)m; j += kTopkThreads) {
+            const uint64_t x = sh.cand[j];
+            const uint32_t bin = bin_of(x);
+            int slot = j;
+            for (int q = j - 1; q >= 0; --q) {
+              const uint64_t y = sh.cand[q];
+              if (bin_of(y) != bin) break;
+              slot -= y < x ? 1 : 0;
+            }
+            for (int q = j + 1; q < (int)m; ++q) {
+              const uint64_t y = sh.cand[q];
+              if (bin_of(y) != bin) break;
+              slot += y > x ? 1 : 0;
+            }
+            if (slot < k) {
+              const uint32_t p = ~(uint32_t)x;
+              if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)p;
+              if (a.out_val) a.out_val[out_base + slot] = scores[p];
+            }
+          }
+          done = true;
+        } else if ((int)m <= 1 << (32 - __clz(k - 1))) {
+          to_sort = (int)m;
+        } else {
+          crowded = true;
+        }
+      } else {
+        if (wave == 0) {
+          const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, (uint32_t)k, false);
+          if (lane == 0) {
+            sh.digit = loc.digit;
+            sh.rem = loc.rem;
+            sh.count = loc.count;
+          }
+        }
+        __syncthreads();
+        lowest = bound + (sh.digit << shift);
+        reach = min((1u << shift) - 1u, hi - lowest);
+        want = sh.rem;
+        if (sh.count <= (uint32_t)kWave) {
+#pragma unroll
+          for (int i = 0; i < CAP / kTopkThreads; ++i)
+            if (c[i] && (uint32_t)(c[i] >> 32) - lowest <= reach) sh.near[atomicAdd(&sh.near_n, 1u)] = c[i];
           __syncthreads();
           if (tid < (int)sh.count) {
             const uint64_t x = sh.near[tid];
             uint32_t larger = 0;
             for (int j = 0; j < (int)sh.count; ++j) larger += sh.near[j] > x ? 1u : 0u;
-            if (larger + 1 == sh.rem) sh.cstar = x;
+            if (larger + 1 == want) sh.cstar = x;
           }
           __syncthreads();
           const uint64_t cstar = sh.cstar;
@@ -722,104 +830,100 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
               const uint32_t p = ~(uint32_t)c[i];
               atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
             }
-          resolved = true;
+        } else {
+          crowded = true;
         }
       }
-    }
-    if (!resolved) {
-      // Radix select of the k-th key over the whole row (12, 12 and 8 bits),
-      // then the ties at it in index order.  With fewer than k keys in the row
-      // there is no k-th (the first pass finds no bin): prefix 0, every key.
-      uint32_t prefix = 0, prefix_mask = 0, want = (uint32_t)k;
-#pragma unroll 1
-      for (int pass = 0; pass < 3; ++pass) {
-        const int sft = pass == 0 ? 20 : (pass == 1 ? 8 : 0);
-        const uint32_t dmask = pass == 2 ? 0xffu : 0xfffu;
-        __syncthreads();
-        reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < EPT; ++e)
-          if (key[e] != 0 && (key[e] & prefix_mask) == prefix) lds_add(&sh.bins[(key[e] >> sft) & dmask], 1u);
-        __syncthreads();
-        if (wave == 0) {
-          const Locate loc = wave_locate<kRowBins / kWave>(sh.bins, want, false);
-          if (lane == 0) {
-            sh.digit = loc.digit;
-            sh.rem = loc.rem;
-          }
-        }
-        __syncthreads();
-        if (sh.digit == kNoBin) {
-          want = 0;
-          break;
-        }
-        prefix |= sh.digit << sft;
-        prefix_mask |= dmask << sft;
-        want = sh.rem;
-      }
-      __syncthreads();
-      uint32_t* ties = sh.bins;  // one word per thread
-      ties[tid] = 0;
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        const int p = pos_of(e);
-        if (key[e] > prefix) atomicOr(&sh.bits[p >> 5], 1u << (p & 31));
-        if (key[e] != 0 && key[e] == prefix) atomicOr(&ties[p >> 5], 1u << (p & 31));
-      }
-      __syncthreads();
-      uint32_t word = ties[tid];
-      uint32_t total;
-      const uint32_t before = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[0], total);
-      int take = (int)want - (int)before;  // this word's ties that are chosen, lowest first
-      uint32_t chosen = 0;
-      while (word && take > 0) {
-        chosen |= word & (0u - word);
-        word &= word - 1;
-        --take;
-      }
-      sh.bits[tid] |= chosen;
+      if (crowded) narrow(each_candidate);
+      resolved = true;
     }
   }
-  int chosen_n = k;  // (a sorted output is written by then only with k candidates)
-  if (!done) {
+  if (to_sort == 0 && !resolved) {
+    // More candidates than fit, or too few: from the row, read again.  A bound
+    // that leaves fewer than k (a sample's, or the least finite key's) is
+    // lowered to the finite keys, to -inf, to any key; with fewer than k keys in
+    // the row, every one of them is chosen (lowest 0).
+    // (Opaque to the compiler, which otherwise keeps the element masks of the
+    // first read for this one: 0.8 us on every row.)
+    const float* again = scores;
+    int again_n = n;
+    asm volatile("" : "+s"(again), "+s"(again_n));
+    uint32_t key[EPT];
+    load(again, again_n, key);
+    order(again_n, key);
+#pragma unroll 1
+    for (int step = 0; m < (uint32_t)k; ++step) {
+      want = bound > 1u ? (uint32_t)k - m : 0u;
+      lowest = bound > lo ? lo : (bound > kNegInfKey ? kNegInfKey : bound > 1u ? 1u : 0u);
+      reach = lowest == kNegInfKey || lowest == 0u ? 0u : bound - 1u - lowest;
+      if (lowest == 0u) break;
+      bound = lowest;
+      uint32_t mine = 0;
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) mine += (uint32_t)__popcll(__ballot(key[e] >= bound));
+      if (lane == 0) sh.ws[~step & 1][wave] = mine;  // (the first count was in ws[0])
+      __syncthreads();
+      m = 0;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) m += sh.ws[~step & 1][i];
+    }
+    narrow([&](auto&& f) {
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) f(key[e], pos_of(e));
+    });
+  }
+  const int chosen_n = min((int)m, k);
+  if (!done && to_sort == 0) {
     __syncthreads();
     uint32_t word = sh.bits[tid];
     uint32_t total;
-    uint32_t p = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[1], total);
-    // min(keys in the row, k) bits are set; the bound only guards the buffers.
-    chosen_n = min((int)total, k);
-    while (word) {
-      const uint32_t at = 32u * tid + (uint32_t)__builtin_ctz(word);
-      word &= word - 1;
-      if (p >= (uint32_t)chosen_n) break;
-      if (a.sorted) {
-        sh.cand[p] = composite(float_to_ordered(scores[at]), (int)at);
-      } else {
-        if (a.out_idx) a.out_idx[out_base + p] = start + (int64_t)at;
-        if (a.out_val) a.out_val[out_base + p] = scores[at];
-      }
-      ++p;
-    }
-    if (a.sorted) {
-      int width = 1;
-      while (width < chosen_n) width <<= 1;
-      for (int i = chosen_n + tid; i < width; i += kTopkThreads) sh.cand[i] = 0;
+    uint32_t slot = block_excl_scan<kWaves>((uint32_t)__popc(word), sh.ws[1], total);
+    // (exactly chosen_n bits are set; the bounds below only guard the buffers)
+    if (a.sorted || 4 * chosen_n >= n) {
+      // To be sorted, or dense: a thread takes its own elements' positions, at
+      // the count of the words before theirs and of the bits below.
+      sh.bins[tid] = slot;
       __syncthreads();
-      bitonic_sort_desc<kTopkThreads>(sh.cand, width);
-      for (int i = tid; i < chosen_n; i += kTopkThreads) {
-        const uint32_t at = ~(uint32_t)sh.cand[i];
-        if (a.out_idx) a.out_idx[out_base + i] = start + (int64_t)at;
-        if (a.out_val) a.out_val[out_base + i] = scores[at];
+#pragma unroll 1
+      for (int p = 4 * tid; p < n; p += kStep) {
+        uint32_t bits = sh.bits[p >> 5];
+        slot = sh.bins[p >> 5] + (uint32_t)__popc(bits & ((1u << (p & 31)) - 1u));
+        bits = bits >> (p & 31) & 15u;
+        for (int at = p; bits && slot < (uint32_t)chosen_n; ++at, bits >>= 1) {
+          if ((bits & 1u) == 0) continue;
+          if (a.sorted) {
+            sh.cand[slot] = composite(float_to_ordered(scores[at]), at);
+          } else {
+            if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)at;
+            if (a.out_val) a.out_val[out_base + slot] = scores[at];
+          }
+          ++slot;
+        }
+      }
+    } else {
+      // A thread writes the few bits of its word.
+      for (; word && slot < (uint32_t)chosen_n; ++slot) {
+        const uint32_t at = 32u * tid + (uint32_t)__builtin_ctz(word);
+        word &= word - 1;
+        if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)at;
+        if (a.out_val) a.out_val[out_base + slot] = scores[at];
       }
     }
+    to_sort = chosen_n;
   }
-  // Padding when the row has fewer than k keys.
-  for (int i = chosen_n + tid; i < k; i += kTopkThreads) {
-    if (a.out_idx) a.out_idx[out_base + i] = -1;
-    if (a.out_val) a.out_val[out_base + i] = -__builtin_inff();
+  if (!done && a.sorted) {
+    int width = 1;
+    while (width < to_sort) width <<= 1;
+    for (int i = to_sort + tid; i < width; i += kTopkThreads) sh.cand[i] = 0;
+    __syncthreads();
+    bitonic_sort_desc<kTopkThreads>(sh.cand, width);
+    for (int i = tid; i < chosen_n; i += kTopkThreads) {
+      const uint32_t p = ~(uint32_t)sh.cand[i];
+      if (a.out_idx) a.out_idx[out_base + i] = start + (int64_t)p;
+      if (a.out_val) a.out_val[out_base + i] = scores[p];
+    }
   }
+  pad_row(a, out_base, chosen_n, tid);
 }
 
 template <int EPT>

@@ -1,6 +1,6 @@
 """The one-workgroup row top-k (topk_rows_kernel through metrics.topk) against
 the oracle's stable_topk, bit for bit: the candidate bound from a full and from
-a sampled histogram, its pairwise, binned and radix resolutions, and the
+a sampled histogram, its pairwise, binned and recounted resolutions, and the
 counting-sorted output, at the edges of the kernel's element counts and on rows
 whose scores share an offset, hold outliers, ties or -inf."""
 
@@ -91,3 +91,51 @@ def test_rows_of_all_ones_bits_are_padded(device, length, k, keys) -> None:
             assert idx[r].tolist() == want.tolist(), (r, by_rank)
             np.testing.assert_array_equal(val[r][want >= 0], host[r][want[want >= 0]])
             assert np.isneginf(val[r][want < 0]).all()
+
+
+def _crowded_row(kind: str, length: int, rng) -> np.ndarray:
+    x = rng.normal(size=length).astype(np.float32)
+    if kind == "some_inf":
+        x[rng.random(length) < 0.4] = -np.inf
+    elif kind == "mostly_inf":
+        x[rng.random(length) < 0.95] = -np.inf
+    elif kind == "all_inf":
+        x[:] = -np.inf
+    elif kind == "steps":  # some twenty distinct values
+        x = np.round(x * 3).astype(np.float32)
+    elif kind == "low_nan":  # NaNs that rank below -inf, by their bits
+        x[rng.random(length) < 0.9] = -np.inf
+        at = rng.random(length) < 0.5
+        x[at] = (np.uint32(0xFFC00000) + rng.integers(0, 9, size=int(at.sum())).astype(np.uint32)).view(np.float32)
+    elif kind == "run":  # the top scores next to each other
+        x[length // 3 : length // 3 + length // 4] += np.float32(8)
+    return x
+
+
+def _by_rank(row: np.ndarray) -> np.ndarray:
+    """Positions by (value desc, index asc); NaNs of the sign bit below -inf, the larger pattern last."""
+
+    bits = row.view(np.uint32).astype(np.int64)
+    value = np.where(np.isnan(row), -np.inf, np.where(row == 0, 0.0, row.astype(np.float64)))
+    return np.lexsort((np.arange(row.size), np.where(np.isnan(row), bits, 0), -value))
+
+
+@pytest.mark.parametrize("kind", ["normal", "some_inf", "mostly_inf", "all_inf", "steps", "low_nan", "run"])
+@pytest.mark.parametrize("length,k", [(1000, 1000), (1001, 999), (4096, 2048), (4095, 4094), (5000, 129), (8190, 4096),
+                                      (16384, 16), (24001, 2048), (32768, 256), (32767, 4096)])
+def test_crowded_cuts_match_oracle(device, kind, length, k) -> None:
+    # Cuts at -inf or below, among equal scores inside a bin, and k near the
+    # row: the bound's steps down, the counts inside a bin, and both outputs.
+    print(f"topk crowded kind={kind} L={length} k={k}", flush=True)
+    rng = np.random.default_rng(2 * length + k)
+    host = np.stack([_crowded_row(kind, length, rng) for _ in range(3)])
+    x = torch.from_numpy(host).to(device)
+    for by_rank in (True, False):
+        idx, val = metrics.topk(x, k, sorted=by_rank, return_values=True)
+        idx, val = idx.cpu().numpy(), val.cpu().numpy()
+        for r in range(3):
+            want = _by_rank(host[r])[:k]
+            if not by_rank:
+                want = np.sort(want)
+            assert idx[r].tolist() == want.tolist(), (r, by_rank)
+            np.testing.assert_array_equal(val[r].view(np.uint32), host[r][want].view(np.uint32))
