@@ -1029,9 +1029,18 @@ int32_t prefill_splits(int64_t blocks, int64_t length) {
   return (int32_t)std::max<int64_t>(1, std::min(kPrefillGrid / blocks, units / kPrefillMinUnits));
 }
 
+// fp8 keys of few units in all (64 keys of one query each) leave the multi-query
+// kernel's workgroups a chain of eight units; one query at a time they are
+// spread over every CU, one unit per wave.  Both score a key to the same bits.
+// One query at a time / four: 4 x 1024 7.9 / 12.0 us, 4 x 32768 (2048 units) 9.5
+// / 12.2, 64 x 4096 (4096) 12.2 / 12.6, 12 x 30000 (5628) 15.5 / 13.8, 4 x 131072
+// 19.6 / 13.9.
+constexpr int64_t kPrefillMinFp8Units = 4096;
+
 template <class Tag, class KF>
 int launch_dense(const DenseArgs& a, int64_t sequences, hipStream_t stream) {
-  if (!a.head_ids && a.head_count == kHeads && a.queries_per_keyset >= kPrefillQueries) {
+  if (!a.head_ids && a.head_count == kHeads && a.queries_per_keyset >= kPrefillQueries &&
+      (!KF::kScaled || sequences * ((a.length + 63) / 64) > kPrefillMinFp8Units)) {
     const int64_t keysets = sequences / a.queries_per_keyset;
     const int64_t qblocks = (a.queries_per_keyset + kPrefillQueries - 1) / kPrefillQueries;
     if (keysets * a.queries_per_keyset == sequences && qblocks * keysets <= 0x7fffffffLL) {

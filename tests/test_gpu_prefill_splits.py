@@ -24,13 +24,19 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("batch,queries,length,fp8", [
-    (1, 4, 1023, False),    # fewer units than two runs' minimum
-    (1, 4, 1024, True),     # two runs of eight units
-    (1, 5, 1089, False),    # an idle wave triple, a run of nine units and one of eight
-    (2, 9, 4099, True),     # two key sets, ragged length
-    (3, 130, 2049, False),  # causal limits inside several runs
+    (1, 4, 960, False),      # 15 units: one run
+    (1, 4, 1023, False),     # 16 units: two runs of eight
+    (1, 5, 1088, False),     # 17 units: a run of nine and one of eight; three idle waves in the second block
+    (3, 130, 2049, False),   # causal limits inside several runs
+    (1, 1540, 1100, False),  # 385 blocks: two runs by the units, three by the grid
+    (1, 2100, 4096, False),  # 525 blocks: two runs by the grid, eight by the units
+    (1, 3100, 1100, False),  # 775 blocks: one run by the grid
+    (1, 4, 1024, True),      # fp8 of few units: one query at a time
+    (2, 9, 4099, True),      # two key sets, ragged length, likewise
+    (1, 256, 1024, True),    # 4096 units, the last such; then four at a time: two runs of eight
+    (1, 257, 1024, True),
     (1, 66, 6200, True),
-    (1, 1540, 1100, False), # query blocks alone pass the grid's half: two runs
+    (2, 130, 2049, True),    # two key sets, a unit of one key, causal limits inside several runs
 ])
 def test_runs_equal_single_queries(device, batch, queries, length, fp8) -> None:
     print(f"prefill runs B={batch} Q={queries} L={length} fp8={fp8}", flush=True)
