@@ -760,16 +760,18 @@ constexpr int64_t kF32SplitTiles = 768;  // 16-key tiles the split kernel takes
 // ---------------------------------------------------------------------------
 // The same product for a few thousand keys, where the launch is a chain of
 // latencies: the four waves of a workgroup take 16 heads each, their dims held
-// in registers, against the same 16-key tiles, and their sums of a tile meet
-// in LDS.  The kernel above gives a wave all 64 heads (128 dependent MFMAs)
-// behind a barrier that stages the queries.  4096 keys: 8.0 us above, 4.9 us
-// here (kernel time); 10000: 7.5 against 6.2 us per call; 32768, where each
-// wave's own tile saves re-reading the keys: 10.8 against 11.8 us.
+// in registers, against the same 16-key tiles, and one of them, in turn, adds
+// their dots of a tile in LDS.  It adds them in the order of the kernel above,
+// so a key scores the same bits in a call of any length and batch.  The kernel
+// above gives a wave all 64 heads (128 dependent MFMAs) behind a barrier that
+// stages the queries.  4096 keys: 8.0 us above, 4.9 us here (kernel time);
+// 10000: 7.5 against 6.2 us per call; 32768, where each wave's own tile saves
+// re-reading the keys: 10.8 against 11.8 us.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void dense_scores_f32_split_kernel(const float* q_all, const float* w_all,
                                                                      const float* keys_all, float* out_all, int L,
                                                                      int tiles_per_wg) {
-  __shared__ float sums[2][4][16];
+  __shared__ floatx4 dots[2][4][64];
   const int64_t b = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -789,9 +791,11 @@ __global__ __launch_bounds__(256) void dense_scores_f32_split_kernel(const float
   const float4* qp = reinterpret_cast<const float4*>(q_all + (b * kHeads + 16 * wave + r) * kHeadDim + 32 * g);
 #pragma unroll
   for (int c = 0; c < 8; ++c) qv[c] = qp[c];
-  float w[4];
+  float w[4][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = w_all[b * kHeads + 16 * wave + 4 * g + i];
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[m][i] = w_all[b * kHeads + 16 * m + 4 * g + i];
   for (int tile = t0; tile < t1; ++tile) {
     load_keys(min(tile + 1, t1 - 1), next);
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -802,17 +806,22 @@ __global__ __launch_bounds__(256) void dense_scores_f32_split_kernel(const float
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[c].z, kv[c].z, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[c].w, kv[c].w, acc, 0, 0, 0);
     }
-    float total = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) total = fmaf(w[i], fmaxf(acc[i], 0.f), total);
-    total = reduce_lane_groups(total);
-    float (&part)[4][16] = sums[tile & 1];
-    if (g == 0) part[wave][r] = total;
+    floatx4 (&part)[4][64] = dots[tile & 1];
+    part[wave][lane] = acc;
     // The other buffer's readers are done once every wave is here again.
     __syncthreads();
-    const int key = 16 * tile + r;
-    if (wave == 0 && g == 0 && key < L)
-      out_all[b * (int64_t)L + key] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+    if (wave == (tile & 3)) {
+      float total = 0.f;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const floatx4 d = part[m][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) total = fmaf(w[m][i], fmaxf(d[i], 0.f), total);
+      }
+      total = reduce_lane_groups(total);
+      const int key = 16 * tile + r;
+      if (g == 0 && key < L) out_all[b * (int64_t)L + key] = total;
+    }
 #pragma unroll
     for (int c = 0; c < 8; ++c) kv[c] = next[c];
   }
@@ -1213,9 +1222,12 @@ extern "C" int dsa_full_scores(const void* queries, const float* weights, const 
               (long long)length);
   if (key_dtype == kF32) {
     const int64_t tiles = (length + 15) / 16;
-    if (tiles * batch <= kF32SplitTiles) {
-      // One workgroup per CU.
-      const int64_t per = (tiles * batch + 255) / 256;
+    if (batch <= 256 && tiles * batch <= kF32SplitTiles) {
+      // At most one workgroup per CU, as many for every sequence (rounded up
+      // over the whole batch, 12 x 1024 gave 264 workgroups and a second round:
+      // 10.7 us against 8.0 of the kernel below).
+      const int64_t per_row = std::max<int64_t>(1, 256 / batch);
+      const int64_t per = (tiles + per_row - 1) / per_row;
       hipLaunchKernelGGL(dense_scores_f32_split_kernel, dim3((unsigned)((tiles + per - 1) / per), (unsigned)batch),
                          dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const float*>(queries), weights,
                          static_cast<const float*>(keys), out, (int)length, (int)per);

@@ -59,7 +59,8 @@ int dsa_abi_version(void);
  *   key_scales [batch, ceil(length/128)] fp32, fp8 keys only (else NULL)
  *   out        [batch, length]     fp32
  * Strides between sequences are the dense ones (64*128, 64, length*128,
- * ceil(length/128), length).
+ * ceil(length/128), length).  A key's score has the same bits in a call of any
+ * batch and length.
  * ------------------------------------------------------------------------ */
 int dsa_full_scores(const void* queries, const float* weights, const void* keys,
                     const float* key_scales, float* out, int64_t batch, int64_t length,
