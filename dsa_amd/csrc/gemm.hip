@@ -903,7 +903,13 @@ int launch_narrow(NarrowArgs& a, int64_t batch, const RopeTableArgs& rope, hipSt
 // against 77; 256-token tiles of eight waves, the only ones before, took 95
 // and 96 there, and 89 at 17 to 128 tokens, where 32-token tiles take 46;
 // 64-token tiles take 51 at 200 against 58 with 128-token tiles and 55 with
-// 32-token ones, 128-token tiles 59 at 400 against 61 and 72.
+// 32-token ones, 128-token tiles 59 at 400 against 61 and 72.  At hidden 512,
+// 1024, 2048, 4096 and 7168 no count of 17 to 8192 tokens is slower than the
+// 256-token tiles of eight waves alone (0.23 to 0.82 of their time).
+//
+// Hidden 1000, 256- against 128-token tiles: 2000 tokens (256 tiles of 256 x
+// 256) 63 / 75 us, 4096 (512) 113 / 133, 3000 (384, three quarters of two
+// rounds) 110 / 105; hidden 4040: 2048 tokens 165 / 208, 8192 567 / 742.
 constexpr int64_t kWideMin = 160;
 template <bool kRope>
 int launch_bf16_features(const GemmArgs& a, hipStream_t stream) {
@@ -916,6 +922,10 @@ int launch_bf16_features(const GemmArgs& a, hipStream_t stream) {
                        stream, a, (int)tiles);
     return check_launch("gemm_wide_kernel");
   }
+  // A kdim that is no multiple of 64: the same tiles on eight waves, one
+  // workgroup per CU, where they fill their last round to seven eighths.
+  const int64_t rounds = (tiles + kWideGrid - 1) / kWideGrid;
+  if (8 * tiles >= 7 * rounds * kWideGrid) return launch_bf16<256, 256, 2, 4, kRope, 1>(a, stream);
   if (groups(128, 128) >= kWideMin) return launch_bf16<128, 128, 2, 4, kRope, 1>(a, stream);
   if (groups(128, 64) >= kWideMin) return launch_bf16<128, 64, 2, 2, kRope, 2>(a, stream);
   return launch_bf16<128, 32, 2, 2, kRope, 4>(a, stream);

@@ -160,6 +160,23 @@ def test_wq_tiles_agree(device, kdim, strided) -> None:
     assert ((whole[-80:].double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * scale).all()
 
 
+@pytest.mark.parametrize("tokens", [1791, 1793, 2048])
+def test_wq_tiles_agree_off_64(device, tokens) -> None:
+    # kdim 136: 224 and 256 tiles of 256 x 256 on eight waves, ragged and whole;
+    # slices of 400 tokens take the 128-token tiles.
+    print(f"wq 256-token tiles tokens={tokens}", flush=True)
+    gen = torch.Generator().manual_seed(tokens)
+    module = sidecar.LightningIndexerSidecar(hidden_size=136).to(device=device, dtype=torch.bfloat16).eval()
+    hidden = torch.randn(tokens, 136, generator=gen).to(device, torch.bfloat16)
+    positions = torch.randint(0, 40000, (tokens,), generator=gen).to(device)
+    whole = module._project(hidden, module.wq.weight)
+    rotated = module._project(hidden, module.wq.weight, positions=positions)
+    for a in range(0, tokens, 400):
+        b = min(tokens, a + 400)
+        assert torch.equal(whole[a:b], module._project(hidden[a:b], module.wq.weight)), a
+        assert torch.equal(rotated[a:b], module._project(hidden[a:b], module.wq.weight, positions=positions[a:b])), a
+
+
 def test_partial_sums_past_one_slice(device) -> None:
     # 1100 tokens x 8192 fp32 features in three splits of k: 96 KiB of partial
     # sums a token, so two slices; 131089 keys in one split: two slices as well.
