@@ -227,3 +227,66 @@ def test_fp32_module_keeps_partial_sums_small(device) -> None:
     own = 2 * (queries.numel() + weights.numel()) * 4
     print(f"  peak {peak / 2**20:.0f} MiB, of it results and projections {own / 2**20:.0f} MiB", flush=True)
     assert peak <= own + (64 << 20) + (1 << 20)
+
+
+def _f32_products(hidden, weight):
+    """The product in float64, and a bound on any fp32 summation of it: 2^-20 of the sum of |h w| (under 2^12 terms, each
+    rounded twice at most along a tree of partial sums)."""
+
+    h, w = hidden.double(), weight.double()
+    return h @ w.t(), 2.0**-20 * (h.abs() @ w.abs().t())
+
+
+@pytest.mark.parametrize("kdim", [72, 264, 1096])  # last stage of 8 k; a last split of 8; a last stage of 8 and a short split
+@pytest.mark.parametrize("tokens,features", [(17, 4), (65, 68), (64, 64)])  # a token and a feature past whole tiles
+def test_fp32_weights_on_bf16_rows_with_tails(device, tokens, features, kdim) -> None:
+    print(f"fp32 weights tokens={tokens} features={features} kdim={kdim}", flush=True)
+    gen = torch.Generator().manual_seed(tokens + kdim)
+    wide = torch.full((tokens, kdim + 24), 1e30, dtype=torch.bfloat16)  # past a row: never read into the sums
+    wide[:, :kdim] = torch.randn(tokens, kdim, generator=gen)
+    hidden = wide.to(device)[:, :kdim]
+    weight = (torch.randn(features, kdim, generator=gen) * kdim**-0.5).to(device)
+    ref, bound = _f32_products(hidden, weight)
+    need = int(_lib.query("dsa_project_weights_workspace_bytes", tokens, kdim, features))
+    ws = torch.empty(need, device=device, dtype=torch.uint8)
+    split, whole = torch.empty(tokens, features, device=device), torch.empty(tokens, features, device=device)
+    _lib.call("dsa_project_weights", hidden.data_ptr(), hidden.stride(0), tokens, kdim, weight.data_ptr(), features, 1.0,
+              split.data_ptr(), ws.data_ptr(), need, _stream())
+    _lib.call("dsa_project_gemm", hidden.data_ptr(), _lib.DTYPE_BF16, hidden.stride(0), tokens, kdim, weight.data_ptr(),
+              _lib.DTYPE_F32, features, whole.data_ptr(), features, 1.0, None, 0.0, None, 0, _stream())
+    assert ((split.double() - ref).abs() <= bound).all()
+    assert ((whole.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("tokens,kdim,heads", [(17, 72, 4), (65, 264, 68), (64, 1096, 4), (300, 128, 68)])
+def test_query_batches_of_other_head_counts(device, tokens, kdim, heads) -> None:
+    # The one-call encoder against the plain projection and its epilogue (bit
+    # for bit, as every wq tile adds k in the same order), that projection
+    # against float64 (half a bf16 ulp, 2^-8 of the value, and the sum's error),
+    # and the head weights with their scale, one more rounding.
+    print(f"encode queries gemm tokens={tokens} kdim={kdim} heads={heads}", flush=True)
+    gen = torch.Generator().manual_seed(tokens + heads)
+    hidden = torch.randn(tokens, kdim + 16, generator=gen).to(device, torch.bfloat16)[:, :kdim]
+    wq = (torch.randn(heads * 128, kdim, generator=gen) * kdim**-0.5).to(device, torch.bfloat16)
+    wp = (torch.randn(heads, kdim, generator=gen) * kdim**-0.5).to(device)
+    positions = torch.randint(0, 40000, (tokens,), generator=gen).to(device)
+    scale = float((heads * 128) ** -0.5)
+    q = torch.empty(tokens, heads, 128, device=device, dtype=torch.bfloat16)
+    w = torch.empty(tokens, heads, device=device)
+    need = int(_lib.query("dsa_encode_queries_workspace_bytes", tokens, kdim, heads))
+    ws = torch.empty(need, device=device, dtype=torch.uint8)
+    _lib.call("dsa_encode_queries_gemm", hidden.data_ptr(), hidden.stride(0), tokens, kdim, wq.data_ptr(), heads,
+              wp.data_ptr(), positions.data_ptr(), 10000.0, scale, q.data_ptr(), w.data_ptr(), ws.data_ptr(), need,
+              _stream())
+    plain = torch.empty(tokens, heads * 128, device=device, dtype=torch.bfloat16)
+    _lib.call("dsa_project_gemm", hidden.data_ptr(), _lib.DTYPE_BF16, hidden.stride(0), tokens, kdim, wq.data_ptr(),
+              _lib.DTYPE_BF16, heads * 128, plain.data_ptr(), heads * 128, 1.0, None, 0.0, None, 0, _stream())
+    want = torch.empty_like(q)
+    unused = torch.empty_like(w)
+    _lib.call("dsa_encode_queries_epilogue", plain.data_ptr(), w.data_ptr(), positions.data_ptr(), 64, 10000.0, scale,
+              want.data_ptr(), unused.data_ptr(), tokens, heads, 128, _lib.DTYPE_BF16, _stream())
+    assert torch.equal(q.view(torch.int16), want.view(torch.int16))
+    ref, bound = _f32_products(hidden, wq)
+    assert ((plain.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2 * bound).all()
+    ref, bound = _f32_products(hidden, wp)
+    assert ((w.double() - scale * ref).abs() <= scale * (bound + 2.0**-23 * ref.abs())).all()

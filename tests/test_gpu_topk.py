@@ -97,11 +97,49 @@ def test_ragged_rows_beyond_resident(device, rows) -> None:
 
 
 @pytest.mark.parametrize("kind", ["normal", "ties", "neginf"])
-@pytest.mark.parametrize("rows,length,k", [(1, 16384, 2048), (3, 32768, 2048), (2, 50000, 4096), (1, 262144, 100)])
+@pytest.mark.parametrize("rows,length,k", [
+    (1, 32769, 2048),   # the shortest rows it takes
+    (2, 40003, 300),    # an odd length: the second row starts off 16 bytes
+    (16, 33000, 4096),  # the most rows
+    (2, 50000, 4096),
+    (1, 262144, 100),
+])
 def test_few_long_rows_distributed(device, kind, rows, length, k) -> None:
-    # Index-order top-k of a few long rows takes the distributed select; the
-    # workspace it shares with the decode step is left ready for reuse.
+    # Index-order top-k of a few rows past one workgroup's 32768 entries takes
+    # the distributed select; the workspace it shares with the decode step is
+    # left ready for reuse.
+    assert length >= metrics.DISTRIBUTED_MIN_LENGTH and rows <= metrics.DISTRIBUTED_MAX_ROWS
     print(f"topk distributed kind={kind} rows={rows} L={length} k={k}", flush=True)
+    host = rows_for(kind, rows, length, seed=length + rows)
+    x = torch.from_numpy(host).to(device)
+    for _ in range(2):
+        idx, val = metrics.topk(x, k, sorted=False, return_values=True)
+        idx, val = idx.cpu().numpy(), val.cpu().numpy()
+        for r in range(rows):
+            want = T.topk_index_order(host[r], k)
+            assert idx[r].tolist() == want.tolist(), r
+            np.testing.assert_array_equal(val[r], host[r][want])
+
+
+def test_distributed_rows_off_16_bytes(device) -> None:
+    # A contiguous slice that starts mid-storage is copied to an aligned buffer.
+    print("topk distributed misaligned slice", flush=True)
+    host = rows_for("normal", 3, 40003, seed=9)
+    x = torch.from_numpy(host).to(device)[1:3]
+    assert x.data_ptr() % 16
+    idx, val = metrics.topk(x, 500, sorted=False, return_values=True)
+    idx, val = idx.cpu().numpy(), val.cpu().numpy()
+    for r in range(2):
+        want = T.topk_index_order(host[1 + r], 500)
+        assert idx[r].tolist() == want.tolist(), r
+        np.testing.assert_array_equal(val[r], host[1 + r][want])
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "neginf"])
+@pytest.mark.parametrize("rows,length,k", [(1, 16384, 2048), (3, 32768, 2048)])
+def test_few_rows_of_one_workgroup(device, kind, rows, length, k) -> None:
+    # Index-order top-k of a few rows up to 32768 entries, one workgroup each.
+    print(f"topk few rows kind={kind} rows={rows} L={length} k={k}", flush=True)
     host = rows_for(kind, rows, length, seed=length + rows)
     x = torch.from_numpy(host).to(device)
     for _ in range(2):

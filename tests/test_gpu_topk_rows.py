@@ -42,7 +42,7 @@ def _row(kind: str, length: int, rng) -> np.ndarray:
 def test_rows_match_oracle(device, kind, length, k) -> None:
     print(f"topk rows kind={kind} L={length} k={k}", flush=True)
     rng = np.random.default_rng(length + k)
-    host = np.stack([_row(kind, length, rng) for _ in range(17)])  # 17 rows: past the distributed select
+    host = np.stack([_row(kind, length, rng) for _ in range(17)])
     wide = torch.full((17, length + 3), float("inf"), device=device)
     wide[:, :length] = torch.from_numpy(host)
     x = wide[:, :length]
