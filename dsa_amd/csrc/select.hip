@@ -495,17 +495,23 @@ __device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, ui
 // trip of loads.  Every list holds all of its chunk's keys at or above
 // `origin`, the highest of the lists' lowest bins (a list of the whole chunk
 // misses nothing), so a k-th largest listed key at or above it is the row's.
-// The entries are counted into bins of 2^12 keys over the octave above the
-// origin and of 2^21 keys from there up, and again inside the cut's bin, from
-// the registers, while that holds more than 64 entries (twice at most).  The
+// The entries are counted into fine bins above the origin and coarse bins, an
+// eighth of an octave, from there up, and again inside the cut's bin, from the
+// registers, while that holds more than 64 entries (twice at most).  The
 // entries of the last bin, ranked by every wave for itself, give the cut; more
 // than 64 equal to it are taken in index order.
 // Scores are signed sums, so a cut near zero, where an octave of keys is a
-// sliver of scores, is as common as one in the octave above the origin; the
-// coarse bins hold those with at most one more count.  (Bins over that octave
-// alone sent k of L / 2, and one row in a few at k = 2048, to the general path
-// below, which costs 3 to 6 us more.  Bins that follow the row's range need its
-// largest key before the first count, 0.4 us of latency.)
+// sliver of scores, is as common as one in the octaves above the origin.  An
+// origin above zero leaves half of the keys to bin: the fine bins are of 2^13
+// keys over two octaves.  Below zero they are of 2^14 over one, and the last
+// coarse bin takes what is past the others.  (Coarse bins of a quarter octave
+// in both cases met a hundred and more of a small k's outliers in the cut's
+// bin: 3 x 65536, k 64, 35.9 us, 3 x 131072, k 64, 48.0 and k 128 47.9, against
+// 33.4, 46.1 and 46.8 with these, and 34.8, 46.7 and 47.0 with 12-bit bins and
+// a radix cut.  Fine bins over that octave alone sent k of L / 2, and one row in
+// a few at k = 2048, to the general path below, which costs 3 to 6 us more.
+// Bins that follow the row's range need its largest key before the first
+// count, 0.4 us of latency.)
 // Returns false, before anything is written, when a list is longer than the
 // registers hold or fewer than k keys lie at or above the origin (a list may
 // miss keys).  in_regs: how many of `pre` hold the list's entries then.
@@ -518,10 +524,21 @@ __device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, ui
 // 2048 35.6 -> 37.4 -> 33.1; 5 x 20011 k 2048 18.9 -> 23.2 -> 18.9; 4 x 4096 k
 // 2048 17.4 -> 20.2 -> 16.0, of 100 equal keys each 19.5 -> 24.1 -> 16.8.
 // ---------------------------------------------------------------------------
-constexpr int kFineShift = 12;    // fine bins of 2^12 keys
-constexpr int kFineBins = 2048;   // over 2^23 keys: an octave
-constexpr int kCoarseShift = 21;  // then of 2^21
-constexpr int kCoarseBase = kFineBins - (kFineBins >> (kCoarseShift - kFineShift));
+constexpr uint32_t kZeroKey = 0x80000000u;  // float_to_ordered(0)
+constexpr int kCoarseShift = 20;            // eight bins an octave
+
+// The first count's fine bins: `count` of 2^shift keys; coarse bins start at
+// bin `count`, bin (d >> kCoarseShift) + base for a key d above the origin.
+struct FineBins {
+  int shift;
+  uint32_t count, base;
+};
+constexpr FineBins fine_bins(int shift, uint32_t count) {
+  return FineBins{shift, count, count - (count >> (kCoarseShift - shift))};
+}
+constexpr FineBins kFineAboveZero = fine_bins(13, 2048);  // two octaves
+constexpr FineBins kFineBelowZero = fine_bins(14, 512);   // one
+static_assert(kFineAboveZero.base + (kZeroKey >> kCoarseShift) <= kSelectBins, "every key above zero has a bin");
 
 __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared& sh, BufferRsrc words, uint32_t lbase,
                                                   uint4 (&pre)[kListVecs], int& in_regs, uint32_t list_len,
@@ -595,13 +612,16 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
   uint32_t lowest = max(top_bin << 20, 1u);
   uint32_t reach = 0xffffffffu;
   uint32_t want = kk, crowd;
-  int shift = kFineShift, coarse_shift = kCoarseShift;
-  uint32_t coarse_base = (uint32_t)kCoarseBase;
+  const bool above_zero = lowest >= kZeroKey;
+  int shift = above_zero ? kFineAboveZero.shift : kFineBelowZero.shift;
+  uint32_t fine = above_zero ? kFineAboveZero.count : kFineBelowZero.count;
+  uint32_t base = above_zero ? kFineAboveZero.base : kFineBelowZero.base;
+  constexpr uint32_t kLastBin = kSelectBins - 1;
 #pragma unroll 1
   for (;;) {
     each([&](uint32_t, uint32_t key) {
       const uint32_t d = key - lowest;
-      const uint32_t b = min(d >> shift, (d >> coarse_shift) + coarse_base);
+      const uint32_t b = min(min(d >> shift, (d >> kCoarseShift) + base), kLastBin);
       if (key >= lowest && d <= reach)
         __hip_atomic_fetch_add(&sh.hist[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     });
@@ -619,15 +639,14 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
     crowd = sh.miss;
     want = sh.want;
     if (bin == kNoBin) return false;
-    const bool coarse = bin >= coarse_base + (uint32_t)(kFineBins - kCoarseBase);
-    const int width = coarse ? coarse_shift : shift;
-    lowest += (coarse ? bin - coarse_base : bin) << width;
-    reach = (1u << width) - 1u;
-    if (crowd <= (uint32_t)kWave || width == 0) break;
-    // Again inside the bin, with no coarse bins.
-    shift = max(0, width - 12);
-    coarse_shift = 31;
-    coarse_base = (uint32_t)kSelectBins;
+    const bool coarse = bin >= fine;
+    const int width = coarse ? kCoarseShift : shift;
+    lowest += (coarse ? bin - base : bin) << width;
+    reach = coarse && bin == kLastBin ? 0xffffffffu - lowest : (1u << width) - 1u;
+    if (crowd <= (uint32_t)kWave || reach == 0) break;
+    // Again inside the bin, with bins of one width.
+    shift = max(0, 20 - (int)__clz((int)reach));
+    fine = base = (uint32_t)kSelectBins;
     clear_hist();
     __syncthreads();
   }

@@ -72,10 +72,12 @@ def signed_rows(kind, batch, length, rng):
         x = np.round(x * 8) / 8
     elif kind == "zeros":  # nine keys in ten score zero, where the cut falls
         x[rng.random(x.shape) < 0.9] = 0.0
+    elif kind == "huge":  # lists that end near -1e30 under a cut near 1e30: the last of the coarse bins
+        x = np.where(rng.random(x.shape) < 0.55, 1.0, -1.0) * 1e30 * (1.0 + np.abs(x))
     return x
 
 
-@pytest.mark.parametrize("kind", ["normal", "shifted", "tight", "outlier", "steps", "zeros"])
+@pytest.mark.parametrize("kind", ["normal", "shifted", "tight", "outlier", "steps", "zeros", "huge"])
 @pytest.mark.parametrize(
     "batch,length,k",
     [(1, 1024, 512), (1, 4096, 2048), (2, 2050, 2049), (16, 1024, 1000), (4, 4096, 4096), (3, 5003, 2501), (5, 20011, 2048),
