@@ -496,6 +496,9 @@ constexpr int kNarrowTok = 64;
 constexpr int kNarrowStages = 8;                        // stages of 64 k in flight
 constexpr int kNarrowK = kNarrowStages * kGemmBK;       // most k per workgroup
 
+template <bool kF32>
+constexpr int kNarrowFeat = kF32 ? 64 : 128;
+
 struct NarrowArgs {
   const uint16_t* hidden;
   int64_t hidden_stride;
@@ -508,7 +511,7 @@ struct NarrowArgs {
 
 template <bool kF32>
 __global__ __launch_bounds__(256, 1) void gemm_narrow_kernel(NarrowArgs a, RopeTableArgs rope, int product_blocks) {
-  constexpr int kFeat = kF32 ? 64 : 128;
+  constexpr int kFeat = kNarrowFeat<kF32>;
   constexpr int kWBytes = kF32 ? 4 : 2;
   constexpr int kWRow = kGemmBK * kWBytes;     // weight row bytes per stage
   constexpr int kWLoads = kFeat * kWRow / 16 / 256;
@@ -845,13 +848,19 @@ int launch_bf16(const GemmArgs& a, hipStream_t stream) {
   return check_launch("gemm_bf16_kernel");
 }
 
+template <bool kF32>
+int64_t narrow_ftiles(int64_t features) {
+  return (features + kNarrowFeat<kF32> - 1) / kNarrowFeat<kF32>;
+}
+
 // k per workgroup of the narrow products: as many workgroups as the CUs take at
 // once (a workgroup's registers fill a CU).  At least 192 instead sent some
 // counts into a half-empty second round: encode_keys at 3000 x 1000 (376
 // workgroups against 188) 18.5 -> 13.6 us, 2304 x 2048 16.9 -> 13.9, 300 x 7168
-// 19.4 -> 13.9.
-int32_t narrow_k(int64_t tokens, int64_t kdim) {
-  const int64_t tiles = (tokens + kNarrowTok - 1) / kNarrowTok;
+// 19.4 -> 13.9.  Feature tiles count as well: without them 8192 fp32 features took
+// 137 us at 200 x 2048 and 582 at 1000 x 2048, now 92 and 352.
+int32_t narrow_k(int64_t tokens, int64_t kdim, int64_t ftiles) {
+  const int64_t tiles = (tokens + kNarrowTok - 1) / kNarrowTok * ftiles;
   int64_t kper = kNarrowK;
   while (kper > 2 * kGemmBK && tiles * ((kdim + kper / 2 - 1) / (kper / 2)) <= 256) kper /= 2;
   return (int32_t)kper;
@@ -862,16 +871,16 @@ int32_t narrow_k(int64_t tokens, int64_t kdim) {
 // 4096 tokens, hidden 2048, would leave 512 MiB, of 65000 tokens 8 GiB); longer
 // batches take a launch per slice.
 constexpr int64_t kNarrowParts = int64_t(64) << 20;
-int64_t narrow_slice(int64_t tokens, int64_t kdim, int64_t features) {
-  const int64_t kper = narrow_k(tokens, kdim);
+int64_t narrow_slice(int64_t tokens, int64_t kdim, int64_t features, int64_t ftiles) {
+  const int64_t kper = narrow_k(tokens, kdim, ftiles);
   const int64_t token_bytes = (kdim + kper - 1) / kper * features * (int64_t)sizeof(float);
   const int64_t most = std::max<int64_t>(kNarrowParts / token_bytes / kNarrowTok, 1) * kNarrowTok;
   return std::min(tokens, most);
 }
 
-int64_t narrow_parts_bytes(int64_t tokens, int64_t kdim, int64_t features) {
-  const int64_t kper = narrow_k(tokens, kdim);
-  return (kdim + kper - 1) / kper * narrow_slice(tokens, kdim, features) * features * (int64_t)sizeof(float);
+int64_t narrow_parts_bytes(int64_t tokens, int64_t kdim, int64_t features, int64_t ftiles) {
+  const int64_t kper = narrow_k(tokens, kdim, ftiles);
+  return (kdim + kper - 1) / kper * narrow_slice(tokens, kdim, features, ftiles) * features * (int64_t)sizeof(float);
 }
 
 // Partial sums of a narrow product over the slice of a.tokens (of `batch`, from
@@ -879,11 +888,10 @@ int64_t narrow_parts_bytes(int64_t tokens, int64_t kdim, int64_t features) {
 // nullable) beside it.
 template <bool kF32>
 int launch_narrow(NarrowArgs& a, int64_t batch, const RopeTableArgs& rope, hipStream_t stream) {
-  constexpr int kFeat = kF32 ? 64 : 128;
-  a.kper = narrow_k(batch, a.kdim);
+  const int64_t ftiles = narrow_ftiles<kF32>(a.features);
+  a.kper = narrow_k(batch, a.kdim, ftiles);
   a.splits = (a.kdim + a.kper - 1) / a.kper;
-  const int64_t blocks = (int64_t)a.splits * ((a.features + kFeat - 1) / kFeat) *
-                         ((a.tokens + kNarrowTok - 1) / kNarrowTok);
+  const int64_t blocks = a.splits * ftiles * ((a.tokens + kNarrowTok - 1) / kNarrowTok);
   const int64_t grid = blocks + (rope.table ? rope_table_blocks(rope.tokens) : 0);
   if (grid > 0x7fffffffLL) return fail(DSA_STATUS_INVALID_ARGUMENT, "problem too large");
   hipLaunchKernelGGL(gemm_narrow_kernel<kF32>, dim3((unsigned)grid), dim3(256), 0, stream, a, rope, (int)blocks);
@@ -997,7 +1005,8 @@ extern "C" int dsa_project_gemm(const void* hidden, int32_t hidden_dtype, int64_
 }
 
 extern "C" int64_t dsa_project_weights_workspace_bytes(int64_t tokens, int64_t kdim, int64_t features) {
-  return tokens > 0 && kdim > 0 && features > 0 ? narrow_parts_bytes(tokens, kdim, features) : 0;
+  if (tokens <= 0 || kdim <= 0 || features <= 0) return 0;
+  return narrow_parts_bytes(tokens, kdim, features, narrow_ftiles<true>(features));
 }
 
 // Shared by the two entry points below: weights_proj's partial sums (with the
@@ -1010,7 +1019,7 @@ static int project_weights(const GemmArgs& a, const float* weight, int64_t featu
   DSA_REQUIRE(reinterpret_cast<uintptr_t>(weight) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
               "the fp32 weights and their output must be 16-byte aligned");
   DSA_REQUIRE((int64_t)a.tokens * features * 4 < (int64_t(1) << 31), "the fp32 output must be below 2 GiB");
-  const int64_t slice = narrow_slice(a.tokens, a.kdim, features);
+  const int64_t slice = narrow_slice(a.tokens, a.kdim, features, narrow_ftiles<true>(features));
   for (int64_t t0 = 0; t0 < a.tokens; t0 += slice) {
     NarrowArgs w = {};
     w.hidden = a.hidden + t0 * a.hidden_stride;
@@ -1053,12 +1062,13 @@ extern "C" int dsa_project_weights(const void* hidden, int64_t hidden_stride, in
 
 extern "C" int64_t dsa_encode_queries_workspace_bytes(int64_t tokens, int64_t kdim, int64_t heads) {
   if (tokens <= 0 || kdim <= 0 || heads <= 0) return 0;
-  return dsa_project_gemm_workspace_bytes(tokens) + narrow_parts_bytes(tokens, kdim, heads);
+  return dsa_project_gemm_workspace_bytes(tokens) +
+         narrow_parts_bytes(tokens, kdim, heads, narrow_ftiles<true>(heads));
 }
 
 extern "C" int64_t dsa_encode_keys_workspace_bytes(int64_t tokens, int64_t kdim, int64_t dim) {
   if (tokens <= 0 || kdim <= 0 || dim <= 0) return 0;
-  return std::max(tokens * dim * 2, tokens > 16 && dim == kHeadDim ? narrow_parts_bytes(tokens, kdim, dim) : 0);
+  return std::max(tokens * dim * 2, tokens > 16 && dim == kHeadDim ? narrow_parts_bytes(tokens, kdim, dim, 1) : 0);
 }
 
 extern "C" int dsa_encode_queries_gemm(const void* hidden, int64_t hidden_stride, int64_t tokens, int64_t kdim,
@@ -1113,7 +1123,7 @@ int launch_encode_keys_gemm(const void* hidden, int64_t hidden_stride, int64_t t
   DSA_REQUIRE(((tokens - 1) * hidden_stride + kdim) * 2 < (int64_t(1) << 31) &&
                   kHeadDim * kdim * 2 < (int64_t(1) << 31),
               "hidden and wk must each be below 2 GiB");
-  const int64_t slice = narrow_slice(tokens, kdim, kHeadDim);
+  const int64_t slice = narrow_slice(tokens, kdim, kHeadDim, 1);
   for (int64_t t0 = 0; t0 < tokens; t0 += slice) {
     NarrowArgs w = {};
     w.hidden = static_cast<const uint16_t*>(hidden) + t0 * hidden_stride;

@@ -227,6 +227,19 @@ def apply_noninterleaved_rope(x: torch.Tensor, positions: torch.Tensor, *, theta
     return out
 
 
+def _split_fp32(tokens: int, kdim: int, features: int) -> bool:
+    """Whether bf16 hidden states meet fp32 weights with k split over workgroups (``dsa_project_weights``: partial sums
+    and a launch that adds them) or in one launch (``dsa_project_gemm``).  Split unless the one launch's workgroups (64
+    features x 16 tokens) run in one round and either k is too short to pay for a second launch or the features alone
+    leave no CUs to split k over.  One launch / split, us a call: 64 features 1000 x 256 7.5 / 8.9, 64 x 2048 19.6 / 9.5;
+    8192 features 17 x 2048 20.5 / 29.9, 64 x 2048 37.8 / 31.6, 2048 x 2048 1074 / 706.  At k 1024 the split is 12.1 / 9.3
+    by itself, but the encoders of an fp32 module wait for the host there, 64 tokens 71 / 78."""
+
+    tiles = -(-features // 64)
+    one_round = tiles * -(-tokens // 16) <= 256
+    return not (one_round and (kdim <= 1024 or tiles * -(-tokens // 64) >= 128))
+
+
 class LightningIndexerSidecar(nn.Module):
     """The indexer sidecar (reference sidecar.py:31-121): same constructor,
     parameters and initialisation; the encoders' epilogues run in HIP."""
@@ -303,7 +316,8 @@ class LightningIndexerSidecar(nn.Module):
         if kdim % 8 or features % 4:
             raise ValueError("sidecar projections need a hidden width that is a multiple of 8 and a multiple of "
                              "4 output features")
-        if w.dtype == torch.float32 and hidden.dtype == torch.bfloat16 and positions is None:
+        if (w.dtype == torch.float32 and hidden.dtype == torch.bfloat16 and positions is None
+                and _split_fp32(tokens, kdim, features)):
             need = int(_lib.query("dsa_project_weights_workspace_bytes", tokens, kdim, features))
             ws = torch.empty(need, device=hidden.device, dtype=torch.uint8)
             _lib.call("dsa_project_weights", _lib.ptr(flat), flat.stride(0), tokens, kdim, _lib.ptr(w), features,

@@ -290,3 +290,24 @@ def test_query_batches_of_other_head_counts(device, tokens, kdim, heads) -> None
     assert ((plain.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2 * bound).all()
     ref, bound = _f32_products(hidden, wp)
     assert ((w.double() - scale * ref).abs() <= scale * (bound + 2.0**-23 * ref.abs())).all()
+
+
+@pytest.mark.parametrize("tokens,features,kdim,split", [
+    (17, 8192, 1032, False),   # 128 feature tiles, one round of the unsplit product
+    (33, 8192, 520, True),     # a second round
+    (256, 1024, 1024, False),  # one round, short k
+    (257, 1024, 1024, True),
+    (256, 1024, 1032, True),   # one round, k past 1024
+])
+def test_fp32_weights_split_or_not(device, tokens, features, kdim, split) -> None:
+    print(f"fp32 weights dispatch tokens={tokens} features={features} kdim={kdim}", flush=True)
+    assert sidecar._split_fp32(tokens, kdim, features) == split
+    gen = torch.Generator().manual_seed(tokens + features)
+    module = sidecar.LightningIndexerSidecar(hidden_size=kdim)
+    hidden = torch.randn(tokens, kdim, generator=gen).to(device, torch.bfloat16)
+    weight = (torch.randn(features, kdim, generator=gen) * kdim**-0.5).to(device)
+    ref, bound = _f32_products(hidden, weight)
+    out = module._project(hidden, weight, fp32=True)
+    scaled = module._project(hidden, weight, fp32=True, scale=0.25)
+    assert ((out.double() - ref).abs() <= bound).all()
+    assert torch.equal(scaled, 0.25 * out)
