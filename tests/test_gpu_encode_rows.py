@@ -181,7 +181,7 @@ def test_partial_sums_past_one_slice(device) -> None:
     # 1100 tokens x 8192 fp32 features in three splits of k: 96 KiB of partial
     # sums a token, so two slices; 131089 keys in one split: two slices as well.
     gen = torch.Generator().manual_seed(41)
-    tokens, kdim, features = 1100, 264, 8192
+    tokens, kdim, features = 1100, 1032, 8192
     print(f"project weights slices tokens={tokens} kdim={kdim} features={features}", flush=True)
     hidden = torch.randn(tokens, kdim, generator=gen).to(device, torch.bfloat16)
     weight = (torch.randn(features, kdim, generator=gen) * kdim**-0.5).to(device)
