@@ -507,11 +507,13 @@ __device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, ui
 // coarse bin takes what is past the others.  (Coarse bins of a quarter octave
 // in both cases met a hundred and more of a small k's outliers in the cut's
 // bin: 3 x 65536, k 64, 35.9 us, 3 x 131072, k 64, 48.0 and k 128 47.9, against
-// 33.4, 46.1 and 46.8 with these, and 34.8, 46.7 and 47.0 with 12-bit bins and
-// a radix cut.  Fine bins over that octave alone sent k of L / 2, and one row in
-// a few at k = 2048, to the general path below, which costs 3 to 6 us more.
+// 32.7, 44.9 and 45.7 with these, and 34.6, 46.7 and 47.0 with 12-bit bins and
+// a radix cut.  Fine bins over one octave alone sent k of L / 2, and one row in
+// a few at k = 2048, to the general path below, which costs 5 to 8 us more.
 // Bins that follow the row's range need its largest key before the first
-// count, 0.4 us of latency.)
+// count, 0.4 us of latency.)  A count is bound by its instructions: one compare
+// per key, not two, took 0.3 to 1.1 us off a call, and a counter of its own for
+// each lane's uncounted keys, in place of a branch, added 0.3.
 // Returns false, before anything is written, when a list is longer than the
 // registers hold or fewer than k keys lie at or above the origin (a list may
 // miss keys).  in_regs: how many of `pre` hold the list's entries then.
@@ -520,9 +522,10 @@ __device__ __forceinline__ uint4 load_scores(BufferRsrc words, uint32_t base, ui
 // VALU instructions a wave, one wave per SIMD; each further count adds a
 // microsecond.  Whole decode calls, MI355X, with 12-bit bins and a radix cut ->
 // with bins over one octave and the general path beyond -> this: 1 x 4096 k 256
-// 15.0 -> 13.4 -> 13.6 us; 5 x 20011 k 256 17.8 -> 16.5 -> 16.7; 16 x 32768 k
-// 2048 35.6 -> 37.4 -> 33.1; 5 x 20011 k 2048 18.9 -> 23.2 -> 18.9; 4 x 4096 k
-// 2048 17.4 -> 20.2 -> 16.0, of 100 equal keys each 19.5 -> 24.1 -> 16.8.
+// 15.8 -> 13.9 -> 14.0 us, k 2048 16.0 -> 20.0 -> 15.2; 16 x 4096 k 2048 17.0 ->
+// 20.0 -> 15.4; 8 x 8192 k 4096 17.3 -> 24.9 -> 17.2; 5 x 20011 k 256 17.2 -> 15.6
+// -> 15.7, k 2048 19.9 -> 17.1 -> 17.0; 16 x 32768 k 2048 34.8 -> 32.3 -> 32.5; 4 x
+// 4096 k 2048, 100 equal keys each, 19.5 -> 24.1 -> 16.8.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kZeroKey = 0x80000000u;  // float_to_ordered(0)
 constexpr int kCoarseShift = 20;            // eight bins an octave
@@ -609,8 +612,9 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
   // The cut is the want-th largest of the keys in [lowest, lowest + reach].  One
   // copy of the counting code serves every count: a second one beside it cost
   // each call 0.7 us of instruction fetch.
+  // (A key below `lowest` is further than any reach, as reach + lowest < 2^32.)
   uint32_t lowest = max(top_bin << 20, 1u);
-  uint32_t reach = 0xffffffffu;
+  uint32_t reach = 0xffffffffu - lowest;
   uint32_t want = kk, crowd;
   const bool above_zero = lowest >= kZeroKey;
   int shift = above_zero ? kFineAboveZero.shift : kFineBelowZero.shift;
@@ -622,7 +626,7 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
     each([&](uint32_t, uint32_t key) {
       const uint32_t d = key - lowest;
       const uint32_t b = min(min(d >> shift, (d >> kCoarseShift) + base), kLastBin);
-      if (key >= lowest && d <= reach)
+      if (d <= reach)
         __hip_atomic_fetch_add(&sh.hist[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     });
     __syncthreads();
@@ -696,7 +700,7 @@ __device__ __forceinline__ bool select_lists_fast(const ListArgs& a, ListShared&
     return true;
   }
   each([&](uint32_t s, uint32_t key) {
-    if (key >= lowest && key - lowest <= reach)
+    if (key - lowest <= reach)
       sh.cands[__hip_atomic_fetch_add(&sh.crowd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)] =
           select_composite(key, j * ck + s);
   });
