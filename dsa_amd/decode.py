@@ -4,9 +4,11 @@ The reference times this step as ``_full_score_kernel`` followed by
 ``torch.topk(scores, K, sorted=False)`` (reference
 scripts/benchmark_progressive_dsa.py:117-123), and defines the selection as
 ``stable_topk`` (metrics.py:9-22).  ``indexer_topk`` runs the whole step as
-three HIP launches over the full GPU (scoring with a per-row score histogram,
-candidate gather, exact resolve) and returns the stable_topk index set of every
-sequence in ascending index order.
+two HIP launches over the full GPU (scoring that lists each chunk's best keys,
+and an exact select over the lists), or three where the lists do not fit the
+selection (scoring with a per-row score histogram, candidate gather, exact
+resolve), and returns the stable_topk index set of every sequence in ascending
+index order.
 """
 
 from __future__ import annotations
