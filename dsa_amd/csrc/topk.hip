@@ -463,14 +463,15 @@ __global__ __launch_bounds__(THREADS) void topk_kernel(TopkArgs a) {
 //
 // 512 rows of 32768, k = 2048, index order: 68 us -> 32 us (two rounds of
 // one workgroup per CU: 128 registers past 16384 elements); 100 rows of 16384:
-// 16.9 -> 11.0; one row of 32768, k = 2048, sorted: 42.5 -> 14.9 us, of 4096:
-// 26.8 -> 9.6 us (the bitonic sort took 66 barriers).  Of 288 shapes (rows of
+// 16.9 -> 11.0; one row of 32768, k = 2048, sorted: 42.8 -> 12.3 us, of 4096:
+// 26.5 -> 7.5 us (the bitonic sort took 66 barriers).  Of 516 shapes (rows of
 // random, bf16, tied, constant and partly -inf scores) none is slower than with
 // topk_kernel or the distributed select.
 // ---------------------------------------------------------------------------
 constexpr int kRowBins = 4096;
 constexpr int kRowPairs = 128;       // candidates ranked pairwise
 constexpr uint32_t kNegInfKey = 0x007fffffu;  // float_to_ordered(-inf)
+constexpr uint32_t kZeroKey = 0x80000000u;    // float_to_ordered(0)
 
 template <int CAP>
 struct RowShared {
@@ -599,7 +600,9 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
         lo = min(lo, sh.wave_lo[i]);
         hi = max(hi, sh.wave_hi[i]);
       }
-      lo = min(lo, hi);
+      // (the same in every lane: kept in scalar registers, of which there are plenty)
+      hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
+      lo = min((uint32_t)__builtin_amdgcn_readfirstlane((int)lo), hi);
       // Candidates: the m keys at or above `bound`.
       bound = n > k ? lo : 1u;  // (n <= k: some elements have no key)
       if (n > k && lo < hi) {
@@ -620,7 +623,7 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
           if (lane == 0) sh.digit = loc.digit == kNoBin ? 0u : loc.digit;  // (fewer finite keys: all of them)
         }
         __syncthreads();
-        bound += sh.digit << shift;
+        bound += (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.digit) << shift;
         reinterpret_cast<uint4*>(sh.bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
       }
       uint32_t mine = 0;
@@ -637,6 +640,7 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
         m += c;
       }
       at = __builtin_amdgcn_readfirstlane(at);
+      m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
       if (candidates()) {
 #pragma unroll
         for (int e = 0; e < EPT; ++e) {
@@ -675,8 +679,8 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
         }
       }
       __syncthreads();
-      lowest += sh.digit << shift;
-      want = sh.rem;
+      lowest += (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.digit) << shift;
+      want = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.rem);
       reach = min((1u << shift) - 1u, end - lowest);
     }
     __syncthreads();
@@ -731,8 +735,21 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
       resolved = true;
     } else {
       // Bins from the bound up, over the candidates alone.
+      // Linear in the key, or, for a sorted output of scores on both sides of zero,
+      // in the score: bins of keys are an eighth of an octave there, and a bin
+      // near one holds more than the 64 the sort takes in every other row of k =
+      // n / 2: 64 x 4096, k 2048, 30.7 us against 7.9, 1 x 5000, k 4096, 49.7
+      // against 9.8.  (A span that is no number, or infinite, keeps the key's bins.)
       const int shift = bin_shift(hi - bound);
-      auto bin_of = [&](uint64_t c) { return ((uint32_t)(c >> 32) - bound) >> shift; };
+      const float low_score = ordered_to_float(bound);
+      const float span = ordered_to_float(hi) - low_score;
+      const bool by_score = a.sorted && bound < kZeroKey && hi > kZeroKey && span < __builtin_inff();
+      const float per_score = (float)kRowBins / span;
+      auto bin_of = [&](uint64_t c) {
+        const uint32_t x = (uint32_t)(c >> 32);
+        return by_score ? min((uint32_t)((ordered_to_float(x) - low_score) * per_score), (uint32_t)kRowBins - 1u)
+                        : (x - bound) >> shift;
+      };
       bool crowded = false;
       uint64_t c[CAP / kTopkThreads];
 #pragma unroll
@@ -773,19 +790,13 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
           __syncthreads();
 #pragma unroll 1
           for (int j = tid; j < (int)m; j += kTopkThreads) {
+            // bins[b] is the end of bin b by now, and so bins[b + 1] its start.
             const uint64_t x = sh.cand[j];
             const uint32_t bin = bin_of(x);
-            int slot = j;
-            for (int q = j - 1; q >= 0; --q) {
-              const uint64_t y = sh.cand[q];
-              if (bin_of(y) != bin) break;
-              slot -= y < x ? 1 : 0;
-            }
-            for (int q = j + 1; q < (int)m; ++q) {
-              const uint64_t y = sh.cand[q];
-              if (bin_of(y) != bin) break;
-              slot += y > x ? 1 : 0;
-            }
+            const uint32_t first = bin + 1u < (uint32_t)kRowBins ? sh.bins[bin + 1u] : 0u;
+            const uint32_t end = sh.bins[bin];
+            int slot = (int)first;
+            for (uint32_t q = first; q < end; ++q) slot += sh.cand[q] > x ? 1 : 0;
             if (slot < k) {
               const uint32_t p = ~(uint32_t)x;
               if (a.out_idx) a.out_idx[out_base + slot] = start + (int64_t)p;
@@ -808,9 +819,9 @@ __global__ __launch_bounds__(kTopkThreads, CAP <= 4096 && EPT <= 16 ? 8 : 4) voi
           }
         }
         __syncthreads();
-        lowest = bound + (sh.digit << shift);
+        lowest = bound + ((uint32_t)__builtin_amdgcn_readfirstlane((int)sh.digit) << shift);
         reach = min((1u << shift) - 1u, hi - lowest);
-        want = sh.rem;
+        want = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.rem);
         if (sh.count <= (uint32_t)kWave) {
 #pragma unroll
           for (int i = 0; i < CAP / kTopkThreads; ++i)

@@ -24,8 +24,8 @@ MAX_ROW = 32768
 # A few rows longer than one workgroup takes go, in index order, through the
 # distributed select (every CU works on them) rather than chunks and a merge.
 # Below, one workgroup per row is the faster: 1-16 rows of 16384, k 256 / 2048,
-# 9.8 / 11.0 us against 13.7 us, of 24001 12.6 / 13.8 against 13.9-14.9, of
-# 32768 13.5 / 14.9 against 13.6-15.3, and one launch against three.
+# 9.4 / 10.4 us against 13.7 us, of 24001 11.8 / 12.7 against 13.9-14.9, of
+# 32768 12.1 / 13.3 against 13.6-15.3, and one launch against three.
 DISTRIBUTED_MAX_ROWS = 16
 DISTRIBUTED_MIN_LENGTH = MAX_ROW + 1
 DISTRIBUTED_MAX_LENGTH = 524288

@@ -139,3 +139,32 @@ def test_crowded_cuts_match_oracle(device, kind, length, k) -> None:
                 want = np.sort(want)
             assert idx[r].tolist() == want.tolist(), (r, by_rank)
             np.testing.assert_array_equal(val[r].view(np.uint32), host[r][want].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["normal", "outlier", "infinite", "denormal", "skewed"])
+@pytest.mark.parametrize("length,k", [(4096, 2048), (5000, 4096), (8192, 3000), (20000, 2048)])
+def test_ranked_rows_across_zero(device, kind, length, k) -> None:
+    # Ranked outputs whose scores lie on both sides of zero, binned by score:
+    # values that crowd one bin, spans past the largest float or of denormals,
+    # and infinities, which keep the key's bins.
+    print(f"topk across zero kind={kind} L={length} k={k}", flush=True)
+    rng = np.random.default_rng(3 * length + k)
+    host = rng.normal(loc=0.3, size=(3, length)).astype(np.float32)
+    if kind == "outlier":
+        host[:, 17] = np.float32(1e30)
+    elif kind == "infinite":
+        host[0, 5], host[1, 6], host[2, 7] = np.inf, np.float32(3e38), -np.inf
+        host[1, 8] = np.float32(-3e38)
+    elif kind == "denormal":
+        host = (host * np.float32(1e-39)).astype(np.float32)
+    elif kind == "skewed":
+        host = np.where(host > 0, host, host * np.float32(1e-6)).astype(np.float32)
+        host[:, ::7] = 0.0
+        host[:, 3::7] = -0.0
+    x = torch.from_numpy(host).to(device)
+    idx, val = metrics.topk(x, k, sorted=True, return_values=True)
+    idx, val = idx.cpu().numpy(), val.cpu().numpy()
+    for r in range(3):
+        want = T.stable_topk(host[r], k)
+        assert idx[r].tolist() == want.tolist(), r
+        np.testing.assert_array_equal(val[r].view(np.uint32), host[r][want].view(np.uint32))
