@@ -1040,16 +1040,24 @@ int32_t prefill_splits(int64_t blocks, int64_t length) {
 
 // fp8 keys of few units in all (64 keys of one query each) leave the multi-query
 // kernel's workgroups a chain of eight units; one query at a time they are
-// spread over every CU, one unit per wave.  Both score a key to the same bits.
-// One query at a time / four: 4 x 1024 7.9 / 12.0 us, 4 x 32768 (2048 units) 9.5
-// / 12.2, 64 x 4096 (4096) 12.2 / 12.6, 12 x 30000 (5628) 15.5 / 13.8, 4 x 131072
-// 19.6 / 13.9.
-constexpr int64_t kPrefillMinFp8Units = 4096;
+// spread over every CU.  Both score a key to the same bits.  That pays while
+// every query's workgroups run in one round, up to 16 units each, and the
+// chain is more than half of those eight.  One query at a time / four: 4 x 1024
+// 7.9 / 12.0 us, 4 x 32768 9.5 / 12.2, 64 x 4096 11.9 / 12.3; not one round: 48 x
+// 4096 17.6 / 12.3, 192 x 1024 17.7 / 12.3, 300 x 512 15.0 / 12.0; 17 units and
+// more: 12 x 30000 15.5 / 13.8, 4 x 131072 19.6 / 13.9; four units: 300 x 256 13.0 /
+// 9.6, 21 x 100 10.0 / 9.5.
+constexpr int64_t kPrefillMinFp8Units = 5;
+bool fp8_one_query_at_a_time(int64_t sequences, int64_t length) {
+  const int64_t units = (length + 63) / 64;
+  const int64_t per_wg = dense_units_per_wg(sequences, length);
+  return units >= kPrefillMinFp8Units && per_wg <= 16 && sequences * ((units + per_wg - 1) / per_wg) <= 256;
+}
 
 template <class Tag, class KF>
 int launch_dense(const DenseArgs& a, int64_t sequences, hipStream_t stream) {
   if (!a.head_ids && a.head_count == kHeads && a.queries_per_keyset >= kPrefillQueries &&
-      (!KF::kScaled || sequences * ((a.length + 63) / 64) > kPrefillMinFp8Units)) {
+      !(KF::kScaled && fp8_one_query_at_a_time(sequences, a.length))) {
     const int64_t keysets = sequences / a.queries_per_keyset;
     const int64_t qblocks = (a.queries_per_keyset + kPrefillQueries - 1) / kPrefillQueries;
     if (keysets * a.queries_per_keyset == sequences && qblocks * keysets <= 0x7fffffffLL) {

@@ -31,9 +31,12 @@ pytestmark = pytest.mark.gpu
     (1, 1540, 1100, False),  # 385 blocks: two runs by the units, three by the grid
     (1, 2100, 4096, False),  # 525 blocks: two runs by the grid, eight by the units
     (1, 3100, 1100, False),  # 775 blocks: one run by the grid
-    (1, 4, 1024, True),      # fp8 of few units: one query at a time
+    (1, 300, 256, True),     # fp8 of four units: four queries at a time, one run
+    (1, 4, 257, True),       # five units: one query at a time
+    (1, 4, 1024, True),      # fp8 of few units: likewise
+    (1, 48, 4096, True),     # 3072 units, 288 workgroups one query at a time: four, eight runs
     (2, 9, 4099, True),      # two key sets, ragged length, likewise
-    (1, 256, 1024, True),    # 4096 units, the last such; then four at a time: two runs of eight
+    (1, 256, 1024, True),    # 256 workgroups of 16 units, the last such; then four at a time: two runs of eight
     (1, 257, 1024, True),
     (1, 66, 6200, True),
     (2, 130, 2049, True),    # two key sets, a unit of one key, causal limits inside several runs
