@@ -181,7 +181,7 @@ def cpu_baseline(q, w, keys, k: int, budget_s: float) -> tuple[dict, "object"]:
 def main() -> None:
     args = parse_args()
     if args.gpus != 1:
-        print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported in this build (the path shards by sequence, see DESIGN.md)", file=sys.stderr)
+        print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported in this build (the path shards by sequence)", file=sys.stderr)
         sys.exit(2)
     if args.config == "c3":
         run_c3(args)
