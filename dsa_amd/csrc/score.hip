@@ -1032,10 +1032,15 @@ int launch_dense_m(DenseArgs a, int64_t sequences, hipStream_t stream, hipEvent_
 // took 489, 472 and 159 us at 512 x 32768, 64 x 32768 and 16 x 10916; the
 // runs take 212, 36 and 13 us.
 constexpr int64_t kPrefillGrid = 1536;
+// Twelve to fifteen units in one run are the longest chain of all: where both
+// halves are resident at once they run as two (3 x 64 queries x 960 fp8 keys 18.4
+// -> 12.0 us, 17.5 one query at a time; 2 x 1000, past it, 26.8 -> 29.0).
 constexpr int64_t kPrefillMinUnits = 8;
+constexpr int64_t kPrefillHalves = 12;
 int32_t prefill_splits(int64_t blocks, int64_t length) {
   const int64_t units = (length + 63) / 64;
-  return (int32_t)std::max<int64_t>(1, std::min(kPrefillGrid / blocks, units / kPrefillMinUnits));
+  const int64_t splits = std::max<int64_t>(1, std::min(kPrefillGrid / blocks, units / kPrefillMinUnits));
+  return (int32_t)(splits == 1 && units >= kPrefillHalves && 2 * blocks <= kPrefillGrid / 2 ? 2 : splits);
 }
 
 // fp8 keys of few units in all (64 keys of one query each) leave the multi-query

@@ -24,7 +24,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("batch,queries,length,fp8", [
-    (1, 4, 960, False),      # 15 units: one run
+    (1, 4, 704, False),      # 11 units: one run
+    (1, 4, 768, False),      # 12 units: two halves
+    (1, 9, 960, True),       # 15 units: eight and seven, with fp8 keys one query at a time
+    (3, 64, 960, True),      # and four at a time
+    (1, 1540, 960, False),   # 385 blocks: both halves would not be resident, one run
     (1, 4, 1023, False),     # 16 units: two runs of eight
     (1, 5, 1088, False),     # 17 units: a run of nine and one of eight; three idle waves in the second block
     (3, 130, 2049, False),   # causal limits inside several runs
