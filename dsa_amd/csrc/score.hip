@@ -1037,8 +1037,17 @@ constexpr int64_t kPrefillGrid = 1536;
 // -> 12.0 us, 17.5 one query at a time; 2 x 1000, past it, 26.8 -> 29.0).
 constexpr int64_t kPrefillMinUnits = 8;
 constexpr int64_t kPrefillHalves = 12;
-int32_t prefill_splits(int64_t blocks, int64_t length) {
+// Blocks that see the same keys (no causal limit) and fill their rounds by
+// themselves, one workgroup on each CU a round, gain nothing from runs of short
+// rows: 3/4 full with fewer than 24 units, or 7/8 with fewer than 64, they keep
+// one run.  One / several: 400 blocks x 1344 37.1 / 39.6 us, 500 x 1792 51.2 / 53.2,
+// 675 x 1344 54.0 / 56.2; 400 x 1792 47.6 / 45.9, 500 x 4096 108.4 / 107.4, and 525,
+// a third round of 13, x 1024 40.5 / 37.7.
+int32_t prefill_splits(int64_t blocks, int64_t length, bool causal) {
   const int64_t units = (length + 63) / 64;
+  const int64_t full = (blocks + 255) / 256 * 256;
+  if (!causal && blocks > 384 && ((4 * blocks >= 3 * full && units < 24) || (8 * blocks >= 7 * full && units < 64)))
+    return 1;
   const int64_t splits = std::max<int64_t>(1, std::min(kPrefillGrid / blocks, units / kPrefillMinUnits));
   return (int32_t)(splits == 1 && units >= kPrefillHalves && 2 * blocks <= kPrefillGrid / 2 ? 2 : splits);
 }
@@ -1066,7 +1075,7 @@ int launch_dense(const DenseArgs& a, int64_t sequences, hipStream_t stream) {
     const int64_t keysets = sequences / a.queries_per_keyset;
     const int64_t qblocks = (a.queries_per_keyset + kPrefillQueries - 1) / kPrefillQueries;
     if (keysets * a.queries_per_keyset == sequences && qblocks * keysets <= 0x7fffffffLL) {
-      const int32_t splits = prefill_splits(qblocks * keysets, a.length);
+      const int32_t splits = prefill_splits(qblocks * keysets, a.length, a.causal_offset >= 0);
       hipLaunchKernelGGL((prefill_scores_kernel<Tag, KF, false>), dim3((unsigned)(qblocks * keysets * splits)),
                          dim3(64 * kPrefillQueries), 0, stream, a, (int32_t)qblocks, (int32_t)keysets, splits);
       return check_launch("prefill_scores_kernel");

@@ -32,7 +32,9 @@ pytestmark = pytest.mark.gpu
     (1, 4, 1023, False),     # 16 units: two runs of eight
     (1, 5, 1088, False),     # 17 units: a run of nine and one of eight; three idle waves in the second block
     (3, 130, 2049, False),   # causal limits inside several runs
-    (1, 1540, 1100, False),  # 385 blocks: two runs by the units, three by the grid
+    (1, 1540, 1100, False),  # 385 blocks: causal two runs by the units, three by the grid; without a limit one
+    (1, 1540, 1472, False),  # 23 units: likewise, two runs by the units
+    (1, 1540, 1473, False),  # 24 units: three runs with or without
     (1, 2100, 4096, False),  # 525 blocks: two runs by the grid, eight by the units
     (1, 3100, 1100, False),  # 775 blocks: one run by the grid
     (1, 300, 256, True),     # fp8 of four units: four queries at a time, one run
